@@ -30,6 +30,10 @@ struct RowNormModulate
     float eps;
     const float* shift;
     const float* scale;
+    // Set: out takes the rows' fp16 planes (csrc/dit_split.h, `groups` groups
+    // a row) and meta their shifts instead of the rows themselves.
+    int* meta = nullptr;
+    int groups = 0;
 };
 
 // out = (h + bias) * gate + residual (bias may be null; gate = null takes it as 1).
@@ -60,6 +64,60 @@ struct SwiGlu
     long long out_stride;
     int rows, width;
 };
+
+// fp32 rows split into fp16 planes (csrc/dit_gemm.hip): per 32 values of a
+// row 64 bytes of hi and 64 bytes of lo, rows padded with zeros to a whole
+// number of such groups; meta[row] holds the row's shift and flags.
+struct SplitRows
+{
+    const float* in; // [rows][width], contiguous
+    void* out;       // [rows][groups][128 bytes]
+    int* meta;       // [rows]
+    int rows;
+};
+
+constexpr int kSplitParts = 4;
+
+struct SplitLaunch
+{
+    SplitRows part[kSplitParts];
+    int width, groups;
+};
+
+// One GEMM of split rows: out = epilogue(A W^T).
+struct GemmProblem
+{
+    const void* a;
+    const void* w;
+    const int* meta_a;
+    const int* meta_w;
+    uint32_t lda, ldw; // row strides of the planes in bytes
+    int m, n, groups;
+    void* out;
+    long long ldo; // in elements
+    const float* bias;
+    const float* gate;
+    const void* residual;
+    long long ldr;
+    int twice;
+};
+
+enum GemmEpilogue
+{
+    kGemmStore = 0, // out = y
+    kGemmGate,      // out = (y + bias) * gate + residual, doubled if twice
+    kGemmSwiGlu     // out[:, c] = silu(y[:, c]) * y[:, n / 2 + c]
+};
+
+struct GemmLaunch
+{
+    GemmProblem problem[2]; // video, text (m = 0: none)
+    int tiles[2];           // set by the launch
+    int epilogue;
+};
+
+hipError_t launch_split_rows(const SplitLaunch& p, hipStream_t stream);
+hipError_t launch_split_gemm(const GemmLaunch& p, hipStream_t stream);
 
 hipError_t launch_rmsnorm_modulate(const RowNormModulate& p, hipStream_t stream);
 hipError_t launch_gate_residual(const GateResidual& p, hipStream_t stream);

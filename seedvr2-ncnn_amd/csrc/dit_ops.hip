@@ -15,6 +15,7 @@
 #include <cstdint>
 
 #include "dit_kernels.h"
+#include "dit_split.h"
 
 namespace awa
 {
@@ -123,11 +124,39 @@ __global__ __launch_bounds__(kRowThreads) void ada_prepare_kernel(const void* em
 
 constexpr int kRowChunks = 4; // chunks of 8 a thread keeps in registers (rows up to 8192 wide)
 
+// Largest value and the union of flags over the workgroup.
+__device__ __forceinline__ void block_max(uint32_t& max, int& flags, uint32_t* red)
+{
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+    {
+        const uint32_t m = __shfl_xor(max, off, 64);
+        max = m > max ? m : max;
+        flags |= __shfl_xor(flags, off, 64);
+    }
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0)
+    {
+        red[wave] = max;
+        red[4 + wave] = static_cast<uint32_t>(flags);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 4; w++)
+    {
+        max = red[w] > max ? red[w] : max;
+        flags |= static_cast<int>(red[4 + w]);
+    }
+}
+
 // y = rmsnorm(x) * (scale_a + scale_b) + (shift_a + shift_b), one workgroup
-// per row; the row stays in registers between the two passes.
+// per row; the row stays in registers between the two passes. PLANES: y goes
+// out as fp16 planes for a split GEMM (its scan and a pass over y saved).
+template <bool PLANES>
 __global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const RowNormModulate p)
 {
     __shared__ float red[4];
+    __shared__ uint32_t red_max[8];
     const long long row = blockIdx.x;
     const int chunks = p.width / 8;
     const long long base_in = row * p.in_stride;
@@ -148,12 +177,20 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const Row
     const float mean = block_sum(ss, red) / static_cast<float>(p.width);
     const float inv = 1.f / sqrtf(mean + p.eps);
     const long long base_out = row * p.out_stride;
+    uint32_t max = 0;
+    int flags = 0;
 #pragma unroll
     for (int j = 0; j < kRowChunks; j++)
     {
         const int ch = threadIdx.x + j * kRowThreads;
         if (ch >= chunks)
+        {
+            if (PLANES)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    v[j][e] = 0.f;
             continue;
+        }
         float y[8];
 #pragma unroll
         for (int e = 0; e < 8; e++)
@@ -167,7 +204,30 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const Row
             for (int e = 0; e < 8; e++)
                 y[e] = y[e] * scale[e] + shift[e];
         }
-        store8(p.out, base_out + 8 * ch, p.out_elemsize, y);
+        if (PLANES)
+        {
+            scan8(y, max, flags);
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                v[j][e] = y[e];
+        }
+        else
+            store8(p.out, base_out + 8 * ch, p.out_elemsize, y);
+    }
+    if (PLANES)
+    {
+        block_max(max, flags, red_max);
+        const int s = shift_of(max);
+        if (threadIdx.x == 0)
+            p.meta[row] = (s + kShiftBias) | flags;
+        char* out = static_cast<char*>(p.out) + row * p.groups * kStageBytes;
+#pragma unroll
+        for (int j = 0; j < kRowChunks; j++)
+        {
+            const int k = (threadIdx.x + j * kRowThreads) * 8;
+            if (k < p.groups * kGroup)
+                store_planes(out, k, v[j], s);
+        }
     }
 }
 
@@ -259,7 +319,10 @@ hipError_t launch_rmsnorm_modulate(const RowNormModulate& p, hipStream_t stream)
         return hipSuccess;
     if (p.width % 8 || p.width > 8 * kRowChunks * kRowThreads || p.in_stride % 8 || p.out_stride % 8)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(rmsnorm_modulate_kernel, dim3(p.rows), dim3(kRowThreads), 0, stream, p);
+    if (p.meta)
+        hipLaunchKernelGGL(rmsnorm_modulate_kernel<true>, dim3(p.rows), dim3(kRowThreads), 0, stream, p);
+    else
+        hipLaunchKernelGGL(rmsnorm_modulate_kernel<false>, dim3(p.rows), dim3(kRowThreads), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -14,10 +14,13 @@
 // MLP on video only and returns text as 2 * y_text. Precision follows the
 // block: fp32 blocks keep fp32 activations, weights and GEMMs; bf16 blocks
 // store activations and GEMM weights in bf16 (round to nearest even) and
-// accumulate in fp32. Parameter vectors (biases, gammas, Ada) are fp32.
+// accumulate in fp32. Parameter vectors (biases, gammas, Ada) are fp32. fp32
+// blocks of enough rows run their GEMMs on split operands (csrc/dit_gemm.hip)
+// with the steps after them in the epilogues (forward_split).
 #include <hip/hip_runtime.h>
 #include <hipblaslt/hipblaslt.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -26,6 +29,7 @@
 #include <new>
 #include <string>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "awa_internal.h"
@@ -55,6 +59,11 @@ struct awa_dit_block
     // the branch's Ada vectors [6][hidden] fp32.
     void* ws[2][7] = {};
     float* ada[2] = {nullptr, nullptr};
+    // Split GEMMs (fp32 blocks of enough rows): fp16 planes and shifts of the
+    // activations and of one weight at a time, per branch.
+    bool split = false;
+    void* planes[2][2] = {};   // [branch][activations, weight]
+    int* shifts[2][2] = {};
 };
 
 namespace
@@ -99,6 +108,16 @@ void release(awa_dit_block* b)
             if (p)
                 (void)hipFree(p);
             p = nullptr;
+        }
+    for (int br = 0; br < 2; br++)
+        for (int k = 0; k < 2; k++)
+        {
+            if (b->planes[br][k])
+                (void)hipFree(b->planes[br][k]);
+            if (b->shifts[br][k])
+                (void)hipFree(b->shifts[br][k]);
+            b->planes[br][k] = nullptr;
+            b->shifts[br][k] = nullptr;
         }
     for (float*& p : b->ada)
     {
@@ -293,6 +312,64 @@ int gemm(awa_dit_block* b, const void* x, long long ldx, const void* w, void* y,
     return AWA_OK;
 }
 
+int groups_of(long long width)
+{
+    return static_cast<int>((width + 31) / 32);
+}
+
+// fp32 blocks of at least this many video rows run their GEMMs on split
+// operands; below, the pass that splits the weights (8 bytes an element, about
+// 230 us of a block at hidden 2560, SwiGLU 6912) costs more than it saves.
+// Whole fp32 block, library GEMMs against split ones: 512 rows 826 / 840 us,
+// 1000 rows 1410 / 1006 us, 2304 rows 2867 / 1482 us, 4600 rows 5530 / 2568 us;
+// at hidden 1024 and 512 rows 231 / 285 us.
+constexpr int kSplitMinRows = 768;
+
+bool use_split(const awa_dit_block* b, long long hd)
+{
+    const awa_dit_block_desc& d = b->desc;
+    if (d.precision != AWA_COMPUTE_F32 || b->tokens[0] < kSplitMinRows)
+        return false;
+    // The kernel addresses planes with 32-bit byte offsets.
+    const long long width = std::max({hd, static_cast<long long>(d.hidden), static_cast<long long>(d.mlp_hidden)});
+    const long long rows = std::max({static_cast<long long>(b->tokens[0]), static_cast<long long>(b->tokens[1]), 3 * hd,
+                                     static_cast<long long>(d.hidden), 2LL * d.mlp_hidden});
+    return rows * groups_of(width) * 128 < (1LL << 32);
+}
+
+int allocate_split(awa_dit_block* b, long long hd)
+{
+    const awa_dit_block_desc& d = b->desc;
+    const int gh = groups_of(d.hidden), ga = groups_of(hd), gm = groups_of(d.mlp_hidden);
+    for (int br = 0; br < 2; br++)
+    {
+        const size_t M = static_cast<size_t>(b->tokens[br]);
+        bool ok = true;
+        auto get = [&](auto*& p, size_t bytes) {
+            void* m = nullptr;
+            ok = ok && hipMalloc(&m, bytes) == hipSuccess;
+            if (ok)
+                p = static_cast<std::remove_reference_t<decltype(p)>>(m);
+        };
+        get(b->ada[br], static_cast<size_t>(6) * d.hidden * sizeof(float));
+        get(b->ws[br][kQkv], M * 3 * hd * 4);
+        get(b->ws[br][kAtt], M * hd * 4);
+        get(b->ws[br][kResid], M * d.hidden * 4);
+        get(b->ws[br][kHidden], M * d.mlp_hidden * 4);
+        get(b->planes[br][0], M * std::max({gh, ga, gm}) * 128);
+        get(b->shifts[br][0], M * sizeof(int));
+        get(b->planes[br][1], std::max({static_cast<size_t>(3 * hd) * gh, static_cast<size_t>(d.hidden) * ga,
+                                        static_cast<size_t>(2) * d.mlp_hidden * gh,
+                                        static_cast<size_t>(d.hidden) * gm}) * 128);
+        get(b->shifts[br][1],
+            static_cast<size_t>(std::max({3 * hd, static_cast<long long>(d.hidden), 2LL * d.mlp_hidden})) *
+                sizeof(int));
+        if (!ok)
+            return fail(AWA_ERR_ALLOC, "DiT block workspace allocation failed");
+    }
+    return AWA_OK;
+}
+
 bool aligned16(const void* p)
 {
     return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
@@ -307,6 +384,170 @@ bool branch_weights_valid(const awa_dit_branch_weights* w, bool full)
     if (full && (!w->mlp_gate || !w->mlp_in || !w->mlp_out || !w->ada))
         return false;
     return true;
+}
+
+// AWA with the q/k RMSNorm fused into its gather.
+int attention(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2], hipStream_t stream)
+{
+    const awa_dit_block_desc& d = b->desc;
+    const awa_blob vq = dense3(b->ws[0][kQkv], d.head_dim, 3 * d.heads, b->tokens[0], b->es);
+    const awa_blob tq = dense3(b->ws[1][kQkv], d.head_dim, 3 * d.heads, b->tokens[1], b->es);
+    const awa_blob vo = dense3(b->ws[0][kAtt], d.head_dim, d.heads, b->tokens[0], b->es);
+    const awa_blob to = dense3(b->ws[1][kAtt], d.head_dim, d.heads, b->tokens[1], b->es);
+    awa_qk_norm norm{W[0]->norm_q, W[0]->norm_k, W[1]->norm_q, W[1]->norm_k, d.norm_eps};
+    return awa::forward_fused(b->plan, &vq, &tq, &norm, &vo, &to, d.precision, stream, nullptr);
+}
+
+// One GEMM step of both branches on split operands: the weights are split,
+// then one launch runs the video and (text_rows > 0) the text GEMM. The
+// activations' planes are in place. in2: a second weight of the same size
+// whose rows follow the first's (SwiGLU).
+int split_gemm(awa_dit_block* b, const float* const (&w)[2], const float* const (&w2)[2], int n, int k, int text_rows,
+               awa::GemmLaunch& g, hipStream_t stream)
+{
+    const int groups = groups_of(k);
+    const size_t pitch = static_cast<size_t>(groups) * 128;
+    awa::SplitLaunch s{};
+    s.width = k;
+    s.groups = groups;
+    for (int br = 0; br < 2; br++)
+    {
+        awa::GemmProblem& q = g.problem[br];
+        q.m = br == 0 ? b->tokens[0] : text_rows;
+        if (q.m <= 0)
+            continue;
+        const int first = w2[br] ? n / 2 : n;
+        char* planes = static_cast<char*>(b->planes[br][1]);
+        s.part[2 * br] = {w[br], planes, b->shifts[br][1], first};
+        if (w2[br])
+            s.part[2 * br + 1] = {w2[br], planes + pitch * first, b->shifts[br][1] + first, n - first};
+        q.a = b->planes[br][0];
+        q.w = planes;
+        q.meta_a = b->shifts[br][0];
+        q.meta_w = b->shifts[br][1];
+        q.lda = q.ldw = static_cast<uint32_t>(pitch);
+        q.n = n;
+        q.groups = groups;
+    }
+    DIT_HIP(awa::launch_split_rows(s, stream), "split_rows launch");
+    DIT_HIP(awa::launch_split_gemm(g, stream), "split GEMM launch");
+    return AWA_OK;
+}
+
+// Splits activations of both branches into their planes.
+int split_activations(awa_dit_block* b, int buf, int width, int text_rows, hipStream_t stream)
+{
+    awa::SplitLaunch s{};
+    s.width = width;
+    s.groups = groups_of(width);
+    for (int br = 0; br < 2; br++)
+        s.part[br] = {static_cast<const float*>(b->ws[br][buf]), b->planes[br][0], b->shifts[br][0],
+                      br == 0 ? b->tokens[0] : text_rows};
+    DIT_HIP(awa::launch_split_rows(s, stream), "split_rows launch");
+    return AWA_OK;
+}
+
+// The block on split fp32 GEMMs (csrc/dit_gemm.hip): the same steps, the video
+// and text GEMM of a step in one launch, the bias, gate, residual and SwiGLU in
+// the GEMMs' epilogues and the norm straight into fp16 planes.
+int forward_split(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2], const void* const (&in)[2],
+                  const void* emb, void* const (&out)[2], hipStream_t stream)
+{
+    const awa_dit_block_desc& d = b->desc;
+    const bool last = d.last_layer != 0;
+    const int hidden = d.hidden, hd = d.heads * d.head_dim, mh = d.mlp_hidden;
+    const int text = b->tokens[1];
+    int rc;
+    auto weight = [](const void* p) { return static_cast<const float*>(p); };
+    const float* const none[2] = {nullptr, nullptr};
+    auto norm = [&](int br, const void* x, int shift_row, bool modulate) {
+        awa::RowNormModulate nm{};
+        nm.in = x;
+        nm.in_elemsize = 4;
+        nm.in_stride = hidden;
+        nm.out = b->planes[br][0];
+        nm.out_elemsize = 4;
+        nm.rows = b->tokens[br];
+        nm.width = hidden;
+        nm.eps = d.norm_eps;
+        nm.shift = modulate ? b->ada[br] + static_cast<size_t>(shift_row) * hidden : nullptr;
+        nm.scale = modulate ? b->ada[br] + static_cast<size_t>(shift_row + 1) * hidden : nullptr;
+        nm.meta = b->shifts[br][0];
+        nm.groups = groups_of(hidden);
+        return awa::launch_rmsnorm_modulate(nm, stream);
+    };
+
+    for (int br = 0; br < 2; br++)
+    {
+        const bool modulate = br == 0 || !last;
+        if (modulate)
+            DIT_HIP(awa::launch_ada_prepare(emb, 4, W[br]->ada, b->ada[br], hidden, stream), "ada_prepare launch");
+        DIT_HIP(norm(br, in[br], 0, modulate), "rmsnorm_modulate launch");
+    }
+    {
+        awa::GemmLaunch g{};
+        g.epilogue = awa::kGemmStore;
+        for (int br = 0; br < 2; br++)
+        {
+            g.problem[br].out = b->ws[br][kQkv];
+            g.problem[br].ldo = 3LL * hd;
+        }
+        const float* const w[2] = {weight(W[0]->qkv), weight(W[1]->qkv)};
+        if ((rc = split_gemm(b, w, none, 3 * hd, hidden, text, g, stream)) != AWA_OK)
+            return rc;
+    }
+    if ((rc = attention(b, W, stream)) != AWA_OK)
+        return rc;
+    if ((rc = split_activations(b, kAtt, hd, text, stream)) != AWA_OK)
+        return rc;
+    {
+        awa::GemmLaunch g{};
+        g.epilogue = awa::kGemmGate;
+        for (int br = 0; br < 2; br++)
+        {
+            const bool full = br == 0 || !last;
+            awa::GemmProblem& q = g.problem[br];
+            q.out = full ? b->ws[br][kResid] : out[br];
+            q.ldo = q.ldr = hidden;
+            q.bias = W[br]->proj_out_bias;
+            q.gate = full ? b->ada[br] + static_cast<size_t>(2) * hidden : nullptr;
+            q.residual = in[br];
+            q.twice = !full;
+        }
+        const float* const w[2] = {weight(W[0]->proj_out), weight(W[1]->proj_out)};
+        if ((rc = split_gemm(b, w, none, hidden, hd, text, g, stream)) != AWA_OK)
+            return rc;
+    }
+    const int mlp_text = last ? 0 : text;
+    for (int br = 0; br < (last ? 1 : 2); br++)
+        DIT_HIP(norm(br, b->ws[br][kResid], 3, true), "rmsnorm_modulate launch");
+    {
+        awa::GemmLaunch g{};
+        g.epilogue = awa::kGemmSwiGlu;
+        for (int br = 0; br < 2; br++)
+        {
+            g.problem[br].out = b->ws[br][kHidden];
+            g.problem[br].ldo = mh;
+        }
+        const float* const w[2] = {weight(W[0]->mlp_gate), weight(W[1]->mlp_gate)};
+        const float* const w2[2] = {weight(W[0]->mlp_in), weight(W[1]->mlp_in)};
+        if ((rc = split_gemm(b, w, w2, 2 * mh, hidden, mlp_text, g, stream)) != AWA_OK)
+            return rc;
+    }
+    if ((rc = split_activations(b, kHidden, mh, mlp_text, stream)) != AWA_OK)
+        return rc;
+    awa::GemmLaunch g{};
+    g.epilogue = awa::kGemmGate;
+    for (int br = 0; br < 2; br++)
+    {
+        awa::GemmProblem& q = g.problem[br];
+        q.out = out[br];
+        q.ldo = q.ldr = hidden;
+        q.gate = b->ada[br] + static_cast<size_t>(5) * hidden;
+        q.residual = b->ws[br][kResid];
+    }
+    const float* const w[2] = {weight(W[0]->mlp_out), weight(W[1]->mlp_out)};
+    return split_gemm(b, w, none, hidden, mh, mlp_text, g, stream);
 }
 
 } // namespace
@@ -346,15 +587,27 @@ int awa_dit_block_create(const awa_dit_block_desc* desc, awa_dit_block** out)
         delete b;
         return rc;
     }
+    const long long hd = static_cast<long long>(desc->heads) * desc->head_dim;
+    b->tokens[0] = desc->source_t * desc->source_h * desc->source_w;
+    b->tokens[1] = desc->text_tokens;
+    b->split = use_split(b, hd);
+    if (b->split)
+    {
+        if ((rc = allocate_split(b, hd)) != AWA_OK)
+        {
+            release(b);
+            delete b;
+            return rc;
+        }
+        *out = b;
+        return AWA_OK;
+    }
     if (hipblasLtCreate(&b->lt) != HIPBLAS_STATUS_SUCCESS || hipMalloc(&b->lt_workspace, kGemmWorkspace) != hipSuccess)
     {
         release(b);
         delete b;
         return fail(AWA_ERR_DEVICE, "hipBLASLt handle or workspace creation failed");
     }
-    b->tokens[0] = desc->source_t * desc->source_h * desc->source_w;
-    b->tokens[1] = desc->text_tokens;
-    const long long hd = static_cast<long long>(desc->heads) * desc->head_dim;
     for (int br = 0; br < 2; br++)
     {
         const long long M = b->tokens[br];
@@ -397,9 +650,11 @@ int awa_dit_block_forward(awa_dit_block* b, const awa_dit_branch_weights* video_
     const int hidden = d.hidden;
     const int hd = d.heads * d.head_dim;
     const int mh = d.mlp_hidden;
-    const awa_dit_branch_weights* W[2] = {video_w, text_w};
-    const void* in[2] = {video, text};
-    void* out[2] = {video_out, text_out};
+    const awa_dit_branch_weights* const W[2] = {video_w, text_w};
+    const void* const in[2] = {video, text};
+    void* const out[2] = {video_out, text_out};
+    if (b->split)
+        return forward_split(b, W, in, emb, out, stream);
     int rc;
 
     // Attention half: Ada vectors, norm + Ada in, QKV projection.
@@ -426,16 +681,8 @@ int awa_dit_block_forward(awa_dit_block* b, const awa_dit_branch_weights* video_
                        stream)) != AWA_OK)
             return rc;
     }
-    // AWA with the q/k RMSNorm fused into its gather.
-    {
-        const awa_blob vq = dense3(b->ws[0][kQkv], d.head_dim, 3 * d.heads, b->tokens[0], es);
-        const awa_blob tq = dense3(b->ws[1][kQkv], d.head_dim, 3 * d.heads, b->tokens[1], es);
-        const awa_blob vo = dense3(b->ws[0][kAtt], d.head_dim, d.heads, b->tokens[0], es);
-        const awa_blob to = dense3(b->ws[1][kAtt], d.head_dim, d.heads, b->tokens[1], es);
-        awa_qk_norm norm{video_w->norm_q, video_w->norm_k, text_w->norm_q, text_w->norm_k, d.norm_eps};
-        if ((rc = awa::forward_fused(b->plan, &vq, &tq, &norm, &vo, &to, d.precision, stream, nullptr)) != AWA_OK)
-            return rc;
-    }
+    if ((rc = attention(b, W, stream)) != AWA_OK)
+        return rc;
     for (int br = 0; br < 2; br++)
     {
         const int M = b->tokens[br];

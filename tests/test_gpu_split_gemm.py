@@ -1,0 +1,108 @@
+"""fp32 DiT blocks whose GEMMs run on split operands (two fp16 planes a row,
+csrc/dit_gemm.hip) against the oracle block, at sizes off every tile: rows and
+columns that end inside a tile, widths that are no multiple of the 32 values
+of a stage, one text token.
+
+Tolerance, max|err| / max|ref|: the split keeps 22 bits and the signs of each
+operand (2^-23 of a value, two operands a product) and sums in fp32; over K
+random terms both errors grow like the result, so the fp32 block's bound of
+1e-5 stands as it does for fp32 products.
+"""
+
+import numpy as np
+import pytest
+
+import awa_hip as A
+import oracle as O
+from awa_cases import geometry
+from test_dit_block_oracle import EPS, HEAD_DIM
+from test_gpu_dit_block import DeviceBranch, download_act, upload_act
+
+pytestmark = pytest.mark.gpu
+
+
+def weights(rng, heads, hidden, mlp):
+    hd = heads * HEAD_DIM
+    n = lambda *s, sd=0.05: (rng.standard_normal(s) * sd).astype(np.float32)
+    return O.DitBranchWeights(qkv=n(3 * hd, hidden), proj_out=n(hidden, hd), proj_out_bias=n(hidden, sd=0.1),
+                              mlp_gate=n(mlp, hidden), mlp_in=n(mlp, hidden), mlp_out=n(hidden, mlp),
+                              norm_q=rng.uniform(0.5, 1.5, HEAD_DIM).astype(np.float32),
+                              norm_k=rng.uniform(0.5, 1.5, HEAD_DIM).astype(np.float32), ada=n(6, hidden, sd=0.5))
+
+
+def inputs(seed, grid, text, heads, hidden, mlp):
+    rng = np.random.default_rng(seed)
+    g = geometry(grid + (2, 8, 8, text), False)
+    n = lambda *s: rng.standard_normal(s).astype(np.float32)
+    return g, n(g.source_tokens, hidden), n(text, hidden), n(hidden * 6), weights(rng, heads, hidden, mlp), \
+        weights(rng, heads, hidden, mlp)
+
+
+def run(g, video, text, emb, wv, wt, heads, hidden, mlp, last=False):
+    blk = A.DitBlock(*g.args, g.text_tokens, g.shifted, heads, HEAD_DIM, hidden, mlp, last, A.COMPUTE_F32, EPS)
+    dv, dt = DeviceBranch(wv, 4), DeviceBranch(wt, 4, adjacent_mlp=True)
+    bv, bt, be = upload_act(video, 4), upload_act(text, 4), upload_act(emb, 4)
+    ov, ot = A.DeviceBuffer(video.size * 4), A.DeviceBuffer(text.size * 4)
+    blk.forward(dv.struct, dt.struct, bv.ptr, bt.ptr, be.ptr, ov.ptr, ot.ptr)
+    A.synchronize()
+    out = download_act(ov, video.shape, 4), download_act(ot, text.shape, 4)
+    blk.destroy()
+    return out
+
+
+def off(a, b):
+    return float(np.max(np.abs(a.astype(np.float64) - b)) / np.max(np.abs(b)))
+
+
+@pytest.mark.parametrize("grid,text,heads,hidden,mlp,last", [
+    ((3, 16, 16), 64, 2, 256, 384, False),  # the fewest rows that split; whole stages
+    ((5, 13, 13), 1, 1, 264, 392, False),   # 845 rows; widths 8 over a stage; one text token
+    ((4, 16, 17), 100, 3, 248, 712, True),  # hidden short of a stage; last block
+])
+def test_split_block_matches_oracle(gpu, grid, text, heads, hidden, mlp, last):
+    print(f"case split block {grid} text={text} heads={heads} hidden={hidden} mlp={mlp} last={last}", flush=True)
+    g, video, txt, emb, wv, wt = inputs(31 + hidden, grid, text, heads, hidden, mlp)
+    got = run(g, video, txt, emb, wv, wt, heads, hidden, mlp, last)
+    ref = O.dit_block(g, video, txt, emb, wv, wt, heads, HEAD_DIM, EPS, last)
+    errs = [off(a, b) for a, b in zip(got, ref)]
+    print(f"  rel err video {errs[0]:.3g} text {errs[1]:.3g}", flush=True)
+    assert max(errs) <= 1e-5
+
+
+def test_split_block_rows_of_any_scale(gpu):
+    """Rows of mlp_out scaled by 2^-60 .. 2^60 (exact): every output column
+    keeps the accuracy of its own scale."""
+    print("case split block row scales", flush=True)
+    grid, heads, hidden, mlp = (3, 16, 16), 2, 256, 384
+    g, video, txt, emb, wv, wt = inputs(5, grid, 8, heads, hidden, mlp)
+    scale = np.exp2(np.linspace(-60, 60, hidden).round()).astype(np.float32)
+    for w in (wv, wt):
+        w.mlp_out = w.mlp_out * scale[:, None]
+    got = run(g, video, txt, emb, wv, wt, heads, hidden, mlp)
+    ref = O.dit_block(g, video, txt, emb, wv, wt, heads, HEAD_DIM, EPS, False)
+    for a, b in zip(got, ref):
+        err = np.max(np.abs(a.astype(np.float64) - b), 0) / np.max(np.abs(b), 0)
+        assert np.max(err) <= 1e-5
+
+
+def test_split_block_infinite_and_nan_weights(gpu):
+    """An infinite weight of mlp_out makes its output column infinite with
+    the sign of the product, a NaN makes its column NaN; the others keep
+    their values."""
+    print("case split block inf nan", flush=True)
+    grid, heads, hidden, mlp = (3, 16, 16), 2, 256, 384
+    g, video, txt, emb, wv, wt = inputs(6, grid, 8, heads, hidden, mlp)
+    clean = O.dit_block(g, video, txt, emb, wv, wt, heads, HEAD_DIM, EPS, False)
+    for w in (wv, wt):
+        w.mlp_out[37, 11] = np.inf
+        w.mlp_out[200, 5] = -np.inf
+        w.mlp_out[129, 383] = np.nan
+    got = run(g, video, txt, emb, wv, wt, heads, hidden, mlp)
+    with np.errstate(invalid="ignore"):
+        ref = O.dit_block(g, video, txt, emb, wv, wt, heads, HEAD_DIM, EPS, False)
+    keep = [c for c in range(hidden) if c not in (37, 129, 200)]
+    for a, b, c in zip(got, ref, clean):
+        assert np.all(np.isnan(a[:, 129]))
+        for col in (37, 200):
+            assert np.array_equal(a[:, col].astype(np.float64), b[:, col])
+        assert off(a[:, keep], c[:, keep]) <= 1e-5
