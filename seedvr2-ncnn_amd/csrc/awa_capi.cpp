@@ -1053,10 +1053,9 @@ int awa_pack(const awa_plan* plan, const awa_blob* video_qkv, const awa_blob* te
     const awa::QkvSource vs{video_qkv->data, vl.token_stride, vl.qkv_stride, video_qkv->elemsize};
     const awa::QkvSource ts{text_qkv->data, tl.token_stride, tl.qkv_stride, text_qkv->elemsize};
     HIP_TRY(awa::launch_pack(plan->dev.rows, plan->sequence_tokens, plan->source_tokens, vs, ts, vl.heads,
-                             vl.head_dim, static_cast<float*>(packed->data), packed->cstep, s),
+                             vl.head_dim, static_cast<float*>(packed->data), packed->cstep, plan->dev.cu_seqlens,
+                             cu_count, static_cast<float*>(cu_seqlens->data), s),
             "pack kernel launch");
-    HIP_TRY(awa::launch_cu_seqlens(plan->dev.cu_seqlens, cu_count, static_cast<float*>(cu_seqlens->data), s),
-            "cu_seqlens kernel launch");
     return AWA_OK;
 }
 
@@ -1186,13 +1185,23 @@ int awa_unpack(const awa_plan* plan, const awa_blob* packed, const awa_blob* vid
     if (!is_mat3(*text_out, head_dim, heads, plan->text_tokens))
         return fail(AWA_ERR_INVALID, "invalid text output blob");
     hipStream_t s = as_stream(stream);
-    HIP_TRY(awa::launch_unpack_video(plan->dev.video_positions, plan->source_t, plan->source_h, plan->source_w,
-                                     packed->data, packed->cstep, packed->elemsize, sink, heads, head_dim, s),
-            "unpack video kernel launch");
-    HIP_TRY(awa::launch_unpack_text(plan->dev.text_positions, static_cast<int>(plan->windows.size()),
-                                    plan->text_tokens, packed->data, packed->cstep, packed->elemsize, text_out->data,
-                                    text_out->cstep, text_out->elemsize, heads, head_dim, s),
-            "unpack text kernel launch");
+    awa::UnpackRows u{};
+    u.video_positions = plan->dev.video_positions;
+    u.text_positions = plan->dev.text_positions;
+    u.source_t = plan->source_t;
+    u.source_h = plan->source_h;
+    u.source_w = plan->source_w;
+    u.window_count = static_cast<int>(plan->windows.size());
+    u.text_tokens = plan->text_tokens;
+    u.packed = packed->data;
+    u.packed_row = packed->cstep;
+    u.packed_elemsize = packed->elemsize;
+    u.video = sink;
+    u.text = text_out->data;
+    u.text_row = text_out->cstep;
+    u.text_elemsize = text_out->elemsize;
+    u.row_elems = heads * head_dim;
+    HIP_TRY(awa::launch_unpack(u, s), "unpack kernel launch");
     return AWA_OK;
 }
 

@@ -141,23 +141,33 @@ hipError_t launch_attention_generic(const void* packed_in, long long in_row, int
                                     long long out_row, const int* cu_seqlens_dev, int window_count, int heads,
                                     int head_dim, int sequence_tokens, hipStream_t stream);
 
+// Pack and its cu_seqlens output.
 hipError_t launch_pack(const RowInfo* rows, int sequence_tokens, int source_tokens, const QkvSource& video,
                        const QkvSource& text, int heads, int head_dim, float* packed, long long packed_row,
-                       hipStream_t stream);
-
-hipError_t launch_cu_seqlens(const int* cu_dev, int count, float* out, hipStream_t stream);
+                       const int* cu_dev, int cu_count, float* cu_out, hipStream_t stream);
 
 hipError_t launch_mmrope(const RowInfo* rows, int sequence_tokens, const void* in, long long in_row,
                          int in_elemsize, float* out, long long out_row, int heads, int head_dim, int rope_dim,
                          int rope_pairs, const float* rope_cs, hipStream_t stream);
 
-hipError_t launch_unpack_video(const int* video_positions, int source_t, int source_h, int source_w,
-                               const void* packed, long long packed_row, int packed_elemsize, const VideoSink& out,
-                               int heads, int head_dim, hipStream_t stream);
+// Unpack: video rows to the token grid, text rows averaged over the windows.
+struct UnpackRows
+{
+    const int* video_positions;
+    const int* text_positions;
+    int source_t, source_h, source_w, window_count, text_tokens;
+    const void* packed;
+    long long packed_row;
+    int packed_elemsize;
+    VideoSink video;
+    void* text;
+    long long text_row;
+    int text_elemsize;
+    int row_elems;   // heads * head_dim
+    int text_blocks; // set by the launch
+};
 
-hipError_t launch_unpack_text(const int* text_positions, int window_count, int text_tokens, const void* packed,
-                              long long packed_row, int packed_elemsize, void* out, long long out_row,
-                              int out_elemsize, int heads, int head_dim, hipStream_t stream);
+hipError_t launch_unpack(UnpackRows u, hipStream_t stream);
 
 // Strided element cast between fp32 and bf16 (or same-type copy): element
 // (x, y, z, c, b) at b*nstep + c*cstep + (z*h + y)*w + x on both sides.

@@ -2,12 +2,11 @@
 // Unpack layers, the ordered text mean of the fused path, a generic-head_dim
 // window attention for the staged layer, casts, fills.
 //
-// All of these are HBM-bound byte movers: each thread moves 4 consecutive
-// elements (16 B of fp32 / 8 B of bf16) so that a wave touches contiguous
-// 256-1024 B runs of a row.
+// All of these are HBM-bound byte movers.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <initializer_list>
 
 #include "awa_kernels.h"
 
@@ -41,6 +40,77 @@ __device__ __forceinline__ void store_elem(void* base, long long index, int elem
         static_cast<float*>(base)[index] = v;
     else
         static_cast<uint16_t*>(base)[index] = f32_to_bf16(v);
+}
+
+// Four consecutive elements, 16-byte (fp32) or 8-byte (bf16) aligned.
+__device__ __forceinline__ float4 load4(const void* base, long long index, int elemsize)
+{
+    if (elemsize == 4)
+        return *reinterpret_cast<const float4*>(static_cast<const float*>(base) + index);
+    const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + index);
+    return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
+                       __uint_as_float(w.y & 0xffff0000u));
+}
+
+__device__ __forceinline__ void store4(void* base, long long index, int elemsize, const float4& v)
+{
+    if (elemsize == 4)
+        *reinterpret_cast<float4*>(static_cast<float*>(base) + index) = v;
+    else
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(base) + index) =
+            make_uint2(f32_to_bf16(v.x) | (static_cast<uint32_t>(f32_to_bf16(v.y)) << 16),
+                       f32_to_bf16(v.z) | (static_cast<uint32_t>(f32_to_bf16(v.w)) << 16));
+}
+
+// The staged movers below are HBM-bound. Where head_dim, strides and base
+// addresses allow it, a workgroup takes one row (its table entry is then a
+// scalar) and every thread moves kRowChunks pieces of four elements with all
+// their loads in flight; other layouts go one element (pair) a thread. At the
+// shifted 33-frame layer (4608 packed rows of 7680 fp32, 36 windows) one
+// element a thread took 108 us (Pack), 70 us (MMRoPE) and 41 us (Unpack), rows
+// take 37 us, 46 us and 23 us.
+constexpr int kRowChunks = 8;
+constexpr int kRowSpan = 4 * kBlock; // elements of a row per chunk step
+
+// Pack by rows. cu: the block past the last row writes cu_seqlens.
+__global__ __launch_bounds__(kBlock) void pack_rows_kernel(const RowInfo* rows, int sequence_tokens,
+                                                           int source_tokens, QkvSource video, QkvSource text,
+                                                           int plane, float* packed, long long packed_row,
+                                                           const int* cu, int cu_count, float* cu_out)
+{
+    const int position = blockIdx.x;
+    if (position >= sequence_tokens)
+    {
+        for (int i = threadIdx.x; i < cu_count; i += kBlock)
+            cu_out[i] = static_cast<float>(cu[i]);
+        return;
+    }
+    const int source = rows[position].source;
+    const bool is_video = source < source_tokens;
+    const QkvSource& src = is_video ? video : text;
+    const long long base = static_cast<long long>(is_video ? source : source - source_tokens) * src.token_stride;
+    float* out = packed + position * packed_row;
+    for (int e0 = 4 * threadIdx.x; e0 < 3 * plane; e0 += kRowChunks * kRowSpan)
+    {
+        float4 v[kRowChunks];
+#pragma unroll
+        for (int j = 0; j < kRowChunks; j++)
+        {
+            const int e = e0 + j * kRowSpan;
+            if (e < 3 * plane)
+            {
+                const int qkv = e >= 2 * plane ? 2 : (e >= plane ? 1 : 0);
+                v[j] = load4(src.data, base + qkv * src.qkv_stride + (e - qkv * plane), src.elemsize);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kRowChunks; j++)
+        {
+            const int e = e0 + j * kRowSpan;
+            if (e < 3 * plane)
+                *reinterpret_cast<float4*>(out + e) = v[j];
+        }
+    }
 }
 
 // ---- Pack: packed[p][qkv][head][f] = source row (src/awa/awa_layers.cpp:440-454) ----
@@ -113,6 +183,119 @@ __global__ void mmrope_kernel(const RowInfo* rows, int sequence_tokens, const vo
     out[dst] = x0;
     if (feature + 1 < head_dim)
         out[dst + 1] = x1;
+}
+
+// MMRoPE by rows; the same products and sums as mmrope_kernel.
+__global__ __launch_bounds__(kBlock) void mmrope_rows_kernel(const RowInfo* rows, const void* in, long long in_row,
+                                                             int in_elemsize, float* out, long long out_row, int heads,
+                                                             int head_dim, int rope_dim, int rope_pairs,
+                                                             const float* rope_cs)
+{
+#pragma clang fp contract(off)
+    const int position = blockIdx.x;
+    const RowInfo r = rows[position];
+    const int rotated = 2 * heads * head_dim, row_elems = 3 * heads * head_dim;
+    for (int e0 = 4 * threadIdx.x; e0 < row_elems; e0 += kRowChunks * kRowSpan)
+    {
+        float4 v[kRowChunks];
+        float2 cs[kRowChunks][2];
+#pragma unroll
+        for (int j = 0; j < kRowChunks; j++)
+        {
+            const int e = e0 + j * kRowSpan;
+            if (e >= row_elems)
+                continue;
+            v[j] = load4(in, position * in_row + e, in_elemsize);
+            if (e >= rotated)
+                continue;
+            const int feature = e % head_dim;
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                if (feature + 2 * i < rope_dim)
+                {
+                    const int pair = (feature >> 1) + i;
+                    const int axis = pair / rope_pairs;
+                    const int coord = axis == 0 ? r.ct : (axis == 1 ? r.ch : r.cw);
+                    cs[j][i] =
+                        *reinterpret_cast<const float2*>(rope_cs + (coord * rope_pairs + pair - axis * rope_pairs) * 2);
+                }
+        }
+#pragma unroll
+        for (int j = 0; j < kRowChunks; j++)
+        {
+            const int e = e0 + j * kRowSpan;
+            if (e >= row_elems)
+                continue;
+            if (e < rotated)
+            {
+                const int feature = e % head_dim;
+                const float4 x = v[j];
+                if (feature < rope_dim)
+                {
+                    v[j].x = x.x * cs[j][0].x - x.y * cs[j][0].y;
+                    v[j].y = x.y * cs[j][0].x + x.x * cs[j][0].y;
+                }
+                if (feature + 2 < rope_dim)
+                {
+                    v[j].z = x.z * cs[j][1].x - x.w * cs[j][1].y;
+                    v[j].w = x.w * cs[j][1].x + x.z * cs[j][1].y;
+                }
+            }
+            *reinterpret_cast<float4*>(out + position * out_row + e) = v[j];
+        }
+    }
+}
+
+// Unpack by rows: the first source_tokens workgroups a video row each, the
+// others kBlock pieces of a text row (text_blocks a row).
+__global__ __launch_bounds__(kBlock) void unpack_rows_kernel(UnpackRows u)
+{
+    const int source_tokens = u.source_t * u.source_h * u.source_w;
+    const int block = blockIdx.x;
+    if (block < source_tokens)
+    {
+        const int t = block / (u.source_h * u.source_w);
+        const int spatial = block - t * u.source_h * u.source_w;
+        const int h = spatial / u.source_w;
+        const int w = spatial - h * u.source_w;
+        const long long src = u.video_positions[block] * u.packed_row;
+        const long long dst = t * u.video.ts + h * u.video.hs + w * u.video.ws;
+        for (int e0 = 4 * threadIdx.x; e0 < u.row_elems; e0 += 4 * kRowSpan)
+        {
+            float4 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (e0 + j * kRowSpan < u.row_elems)
+                    v[j] = load4(u.packed, src + e0 + j * kRowSpan, u.packed_elemsize);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (e0 + j * kRowSpan < u.row_elems)
+                    store4(u.video.data, dst + e0 + j * kRowSpan, u.video.elemsize, v[j]);
+        }
+        return;
+    }
+    const int k = (block - source_tokens) / u.text_blocks;
+    const int e = 4 * ((block - source_tokens - k * u.text_blocks) * kBlock + static_cast<int>(threadIdx.x));
+    if (e >= u.row_elems)
+        return;
+    // Window order, kBatch windows' loads at a time (clamped past the last).
+    constexpr int kBatch = 12;
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int w0 = 0; w0 < u.window_count; w0 += kBatch)
+    {
+        float4 v[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; j++)
+            v[j] = load4(u.packed,
+                         u.text_positions[min(w0 + j, u.window_count - 1) * u.text_tokens + k] * u.packed_row + e,
+                         u.packed_elemsize);
+#pragma unroll
+        for (int j = 0; j < kBatch; j++)
+            if (w0 + j < u.window_count)
+                sum.x += v[j].x, sum.y += v[j].y, sum.z += v[j].z, sum.w += v[j].w;
+    }
+    const float n = static_cast<float>(u.window_count);
+    store4(u.text, k * u.text_row + e, u.text_elemsize, make_float4(sum.x / n, sum.y / n, sum.z / n, sum.w / n));
 }
 
 // ---- Unpack video: video[t][h][w][head][f] = packed[video_positions[token]] (awa_layers.cpp:659-676) ----
@@ -603,19 +786,35 @@ hipError_t launch_attention_generic(const void* packed_in, long long in_row, int
     return hipGetLastError();
 }
 
+// The pieces of four elements at every multiple of the strides are aligned.
+bool aligned4(const void* p, int elemsize, std::initializer_list<long long> strides)
+{
+    bool ok = reinterpret_cast<uintptr_t>(p) % (4 * elemsize) == 0;
+    for (long long s : strides)
+        ok = ok && s % 4 == 0;
+    return ok;
+}
+
 hipError_t launch_pack(const RowInfo* rows, int sequence_tokens, int source_tokens, const QkvSource& video,
                        const QkvSource& text, int heads, int head_dim, float* packed, long long packed_row,
-                       hipStream_t stream)
+                       const int* cu_dev, int cu_count, float* cu_out, hipStream_t stream)
 {
+    if (aligned4(packed, 4, {packed_row, head_dim}) &&
+        aligned4(video.data, video.elemsize, {video.token_stride, video.qkv_stride}) &&
+        aligned4(text.data, text.elemsize, {text.token_stride, text.qkv_stride}))
+    {
+        hipLaunchKernelGGL(pack_rows_kernel, dim3(sequence_tokens + 1), dim3(kBlock), 0, stream, rows,
+                           sequence_tokens, source_tokens, video, text, heads * head_dim, packed, packed_row, cu_dev,
+                           cu_count, cu_out);
+        return hipGetLastError();
+    }
     const long long total = static_cast<long long>(sequence_tokens) * 3 * heads * head_dim;
     hipLaunchKernelGGL(pack_kernel, dim3(grid_for(total)), dim3(kBlock), 0, stream, rows, sequence_tokens,
                        source_tokens, video, text, heads, head_dim, packed, packed_row);
-    return hipGetLastError();
-}
-
-hipError_t launch_cu_seqlens(const int* cu_dev, int count, float* out, hipStream_t stream)
-{
-    hipLaunchKernelGGL(cu_seqlens_kernel, dim3(grid_for(count)), dim3(kBlock), 0, stream, cu_dev, count, out);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return e;
+    hipLaunchKernelGGL(cu_seqlens_kernel, dim3(grid_for(cu_count)), dim3(kBlock), 0, stream, cu_dev, cu_count, cu_out);
     return hipGetLastError();
 }
 
@@ -623,32 +822,39 @@ hipError_t launch_mmrope(const RowInfo* rows, int sequence_tokens, const void* i
                          int in_elemsize, float* out, long long out_row, int heads, int head_dim, int rope_dim,
                          int rope_pairs, const float* rope_cs, hipStream_t stream)
 {
+    if (aligned4(in, in_elemsize, {in_row, head_dim}) && aligned4(out, 4, {out_row}))
+    {
+        hipLaunchKernelGGL(mmrope_rows_kernel, dim3(sequence_tokens), dim3(kBlock), 0, stream, rows, in, in_row,
+                           in_elemsize, out, out_row, heads, head_dim, rope_dim, rope_pairs, rope_cs);
+        return hipGetLastError();
+    }
     const long long total = static_cast<long long>(sequence_tokens) * (3 * heads * head_dim / 2);
     hipLaunchKernelGGL(mmrope_kernel, dim3(grid_for(total)), dim3(kBlock), 0, stream, rows, sequence_tokens, in,
                        in_row, in_elemsize, out, out_row, heads, head_dim, rope_dim, rope_pairs, rope_cs);
     return hipGetLastError();
 }
 
-hipError_t launch_unpack_video(const int* video_positions, int source_t, int source_h, int source_w,
-                               const void* packed, long long packed_row, int packed_elemsize, const VideoSink& out,
-                               int heads, int head_dim, hipStream_t stream)
+hipError_t launch_unpack(UnpackRows u, hipStream_t stream)
 {
-    const int row_elems = heads * head_dim;
-    const long long total = static_cast<long long>(source_t) * source_h * source_w * row_elems;
-    hipLaunchKernelGGL(unpack_video_kernel, dim3(grid_for(total)), dim3(kBlock), 0, stream, video_positions,
-                       source_t, source_h, source_w, packed, packed_row, packed_elemsize, out, row_elems);
-    return hipGetLastError();
-}
-
-hipError_t launch_unpack_text(const int* text_positions, int window_count, int text_tokens, const void* packed,
-                              long long packed_row, int packed_elemsize, void* out, long long out_row,
-                              int out_elemsize, int heads, int head_dim, hipStream_t stream)
-{
-    const int row_elems = heads * head_dim;
-    const long long total = static_cast<long long>(text_tokens) * row_elems;
-    hipLaunchKernelGGL(unpack_text_kernel, dim3(grid_for(total)), dim3(kBlock), 0, stream, text_positions,
-                       window_count, text_tokens, packed, packed_row, packed_elemsize, out, out_row, out_elemsize,
-                       row_elems);
+    const long long source_tokens = static_cast<long long>(u.source_t) * u.source_h * u.source_w;
+    if (aligned4(u.packed, u.packed_elemsize, {u.packed_row, u.row_elems}) &&
+        aligned4(u.video.data, u.video.elemsize, {u.video.ts, u.video.hs, u.video.ws}) &&
+        aligned4(u.text, u.text_elemsize, {u.text_row}))
+    {
+        u.text_blocks = (u.row_elems / 4 + kBlock - 1) / kBlock;
+        const long long blocks = source_tokens + static_cast<long long>(u.text_tokens) * u.text_blocks;
+        hipLaunchKernelGGL(unpack_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, u);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(unpack_video_kernel, dim3(grid_for(source_tokens * u.row_elems)), dim3(kBlock), 0, stream,
+                       u.video_positions, u.source_t, u.source_h, u.source_w, u.packed, u.packed_row,
+                       u.packed_elemsize, u.video, u.row_elems);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return e;
+    hipLaunchKernelGGL(unpack_text_kernel, dim3(grid_for(static_cast<long long>(u.text_tokens) * u.row_elems)),
+                       dim3(kBlock), 0, stream, u.text_positions, u.window_count, u.text_tokens, u.packed,
+                       u.packed_row, u.packed_elemsize, u.text, u.text_row, u.text_elemsize, u.row_elems);
     return hipGetLastError();
 }
 

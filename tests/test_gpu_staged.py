@@ -197,3 +197,68 @@ def test_cast_round_trip(gpu):
     expect = A.bf16_bits_to_f32(A.f32_to_bf16_bits(x))
     np.testing.assert_array_equal(read_mat3(b), expect)
     np.testing.assert_array_equal(read_mat3(c), expect)
+
+
+@pytest.mark.parametrize("head_dim,offset", [(128, 0), (128, 1), (12, 0), (12, 3)])
+@pytest.mark.parametrize("elemsize", [4, 2])
+def test_movers_by_rows_and_by_element_agree(gpu, elemsize, head_dim, offset):
+    """Pack, MMRoPE and Unpack on blobs at element offsets that allow and
+    forbid four-element pieces: bit-exact against the oracle's maps, MMRoPE
+    against the aligned call of the same values."""
+    print(f"case movers elemsize={elemsize} head_dim={head_dim} offset={offset}", flush=True)
+    g = geometry((3, 11, 13, 2, 3, 3, 5), True)
+    heads = 4  # channels of whole 16 bytes: cstep = w * h
+    rng = np.random.default_rng(3)
+    rounded = (lambda a: A.bf16_bits_to_f32(A.f32_to_bf16_bits(a)).reshape(a.shape)) if elemsize == 2 else (lambda a: a)
+
+    class Blob:
+        """An fp32 or bf16 Mat(w, h, c) `off` elements into its allocation."""
+
+        def __init__(self, shape, es, off, values=None):
+            self.shape, self.es, self.off, self.n = shape, es, off, int(np.prod(shape))
+            host = np.zeros(self.n + 8, np.float32)
+            if values is not None:
+                host[off:off + self.n] = values.reshape(-1)
+            self.buf = A.DeviceBuffer((self.n + 8) * es)
+            self.buf.upload(A.f32_to_bf16_bits(host) if es == 2 else host)
+            c, h, w = shape
+            self.blob = A.mat(self.buf.ptr + off * es, w, h, c, es, dims=3)
+
+        def read(self):
+            raw = self.buf.download((self.n + 8,), np.uint16 if self.es == 2 else np.float32)
+            v = A.bf16_bits_to_f32(raw) if self.es == 2 else raw
+            return v[self.off:self.off + self.n].reshape(self.shape)
+
+    m = O.build_maps(g)
+    plan = make_plan(g, 6 * (head_dim // 6) if head_dim != 128 else 126)
+    rows, nwin = m.sequence_tokens, m.window_count
+    x = rounded(rng.standard_normal((g.source_tokens + g.text_tokens, 3 * heads, head_dim)).astype(np.float32))
+    video, text = Blob(x[:g.source_tokens].shape, elemsize, offset, x[:g.source_tokens]), \
+        Blob(x[g.source_tokens:].shape, elemsize, offset, x[g.source_tokens:])
+    packed = Blob((rows, 3 * heads, head_dim), 4, offset)
+    cu = DeviceMat(dict(w=nwin + 1, dims=1), nwin + 1, 4)
+    plan.pack(video.blob, text.blob, packed.blob, cu.blob)
+    A.synchronize()
+    vpos, tpos = np.asarray(m.video_positions), np.asarray(m.text_positions).reshape(nwin, -1)
+    got = packed.read()
+    assert np.array_equal(got[vpos], x[:g.source_tokens])
+    assert all(np.array_equal(got[t], x[g.source_tokens:]) for t in tpos)
+    assert np.array_equal(cu.download_raw(), m.cu_seqlens)
+
+    roped, plain = Blob(packed.shape, 4, offset), Blob(packed.shape, 4, 0)
+    same = Blob(packed.shape, 4, 0, got)
+    plan.mmrope(packed.blob, roped.blob)
+    plan.mmrope(same.blob, plain.blob)
+    A.synchronize()
+    assert np.array_equal(roped.read(), plain.read()) and not np.array_equal(plain.read(), got)
+
+    values = rng.standard_normal((rows, heads, head_dim)).astype(np.float32)
+    att = Blob(values.shape, 4, offset, values)
+    vo, to = Blob((g.source_tokens, heads, head_dim), elemsize, offset), Blob((g.text_tokens, heads, head_dim), elemsize, offset)
+    plan.unpack(att.blob, vo.blob, to.blob)
+    A.synchronize()
+    mean = np.zeros((g.text_tokens, heads, head_dim), np.float32)
+    for t in tpos:
+        mean += values[t]
+    assert np.array_equal(vo.read(), rounded(values[vpos]))
+    assert np.array_equal(to.read(), rounded(mean / np.float32(nwin)))
