@@ -167,25 +167,44 @@ int check_plan_uploaded(const awa_plan* plan)
 // their K/V reads.
 constexpr int kXcds = 8;
 
+// Mean keys of a work item from which a layer counts as one of long windows.
+constexpr long long kLongItemKeys = 640;
+constexpr long long kDeviceCus = 256;
+
 // Attention kernel variant per arithmetic and geometry. AWA_COMPUTE_F32_MFMA
 // takes the 8-wave fp32-MFMA pipeline (one workgroup per unit of up to 256
 // rows). The bf16 and the exact-score fp32 kernels take their 8-wave form when
 // its 256-row query blocks leave no more waves idle than 128-row blocks would
 // (each unit's K/V tiles are then staged once instead of once per 128-row
-// block), else the 4-wave form with two workgroups per CU.
-int attention_variant(int compute, const awa_plan& plan)
+// block), else the 4-wave form with two workgroups per CU. Layers of long
+// windows take the 8-wave form in spite of idle waves: staging (K's RoPE, the
+// digit slices) is then a large part of the loop and is halved, while the rows
+// of idle waves cost little. Measured at 24 layers of mixed windows of up to
+// 1720 rows, 4-wave against 8-wave time: 1.28-1.33 where the mean work item
+// has at least 670 keys, 0.93-1.07 at 400-600 keys, 0.86-1.05 below; the
+// 121-frame 720p bf16 layer 4016 / 2776 us, the 49-frame fp32 one 4871 / 3720.
+int attention_variant(int compute, const awa_plan& plan, int heads)
 {
     if (compute == AWA_COMPUTE_F32_MFMA)
         return awa::kVariantWidePipe;
-    long long idle_wide = 0, idle_narrow = 0;
+    long long idle_wide = 0, idle_narrow = 0;         // waves
+    long long items_wide = 0, keys_wide = 0, keys_narrow = 0; // work items, and the keys they walk
     for (const awa::WindowDesc& w : plan.window_descs)
     {
-        const int L = w.video_tokens + plan.text_tokens;
-        const int waves = (L + 31) / 32;
-        idle_wide += (L + awa::kWideQueryRows - 1) / awa::kWideQueryRows * (awa::kWideQueryRows / 32) - waves;
-        idle_narrow += (L + awa::kQueryRows - 1) / awa::kQueryRows * (awa::kQueryRows / 32) - waves;
+        const long long L = w.video_tokens + plan.text_tokens;
+        const long long waves = (L + 31) / 32;
+        const long long wide = (L + awa::kWideQueryRows - 1) / awa::kWideQueryRows;
+        const long long narrow = (L + awa::kQueryRows - 1) / awa::kQueryRows;
+        idle_wide += wide * (awa::kWideQueryRows / 32) - waves;
+        idle_narrow += narrow * (awa::kQueryRows / 32) - waves;
+        items_wide += wide;
+        keys_wide += wide * L;
+        keys_narrow += narrow * L;
     }
-    return idle_wide <= idle_narrow ? awa::kVariantWide : awa::kVariantNarrow;
+    const bool long_windows = keys_wide >= kLongItemKeys * items_wide &&
+                              keys_wide * 200 <= keys_narrow * 112 && // at most 12 % more work per CU
+                              items_wide * heads >= 3 * kDeviceCus;   // the last round stays a small part
+    return idle_wide <= idle_narrow || long_windows ? awa::kVariantWide : awa::kVariantNarrow;
 }
 
 // The variant to launch: attention_variant's choice, or the 4-wave form
@@ -198,7 +217,7 @@ int launch_variant(int compute, const awa_plan& plan, awa::AttentionLaunch& p)
         return fail(AWA_ERR_INVALID, "window of " + std::to_string(plan.max_window_tokens) +
                                          " rows exceeds the attention kernels' " +
                                          std::to_string(awa::kMaxWindowRows - 1) + "-row limit");
-    p.variant = attention_variant(compute, plan);
+    p.variant = attention_variant(compute, plan, plan.work_heads);
     auto lds = [&](int variant, const awa::AttentionLaunch& q) {
         if (compute == AWA_COMPUTE_F32)
             return awa::attention_x_static_lds(variant == awa::kVariantWide) +
