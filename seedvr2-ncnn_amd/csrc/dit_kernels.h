@@ -84,15 +84,18 @@ struct SplitLaunch
     int width, groups;
 };
 
-// One GEMM of split rows: out = epilogue(A W^T).
+// One GEMM: out = epilogue(A W^T); rows of 128-byte stages (bf16, or split
+// planes). out, residual: bf16 or (split) fp32, rows 16-byte aligned.
 struct GemmProblem
 {
     const void* a;
     const void* w;
-    const int* meta_a;
+    const void* w2;    // SwiGLU: the weight of the second half of the columns
+    const int* meta_a; // split: shifts and flags of A's rows and the weights'
     const int* meta_w;
-    uint32_t lda, ldw; // row strides of the planes in bytes
-    int m, n, groups;
+    uint32_t lda, ldw; // row strides in bytes, multiples of 16
+    int m, n, stages;
+    uint32_t last_bytes; // bf16: bytes of a row in its last stage
     void* out;
     long long ldo; // in elements
     const float* bias;
@@ -117,7 +120,7 @@ struct GemmLaunch
 };
 
 hipError_t launch_split_rows(const SplitLaunch& p, hipStream_t stream);
-hipError_t launch_split_gemm(const GemmLaunch& p, hipStream_t stream);
+hipError_t launch_gemm(const GemmLaunch& p, bool split, hipStream_t stream);
 
 hipError_t launch_rmsnorm_modulate(const RowNormModulate& p, hipStream_t stream);
 hipError_t launch_gate_residual(const GateResidual& p, hipStream_t stream);

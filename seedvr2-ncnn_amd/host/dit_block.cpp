@@ -16,7 +16,7 @@
 // store activations and GEMM weights in bf16 (round to nearest even) and
 // accumulate in fp32. Parameter vectors (biases, gammas, Ada) are fp32. fp32
 // blocks of enough rows run their GEMMs on split operands (csrc/dit_gemm.hip)
-// with the steps after them in the epilogues (forward_split).
+// with the steps after them in the epilogues (forward_grouped).
 #include <hip/hip_runtime.h>
 #include <hipblaslt/hipblaslt.h>
 
@@ -312,6 +312,11 @@ int gemm(awa_dit_block* b, const void* x, long long ldx, const void* w, void* y,
     return AWA_OK;
 }
 
+bool aligned16(const void* p)
+{
+    return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
+}
+
 int groups_of(long long width)
 {
     return static_cast<int>((width + 31) / 32);
@@ -320,21 +325,51 @@ int groups_of(long long width)
 // fp32 blocks of at least this many video rows run their GEMMs on split
 // operands; below, the pass that splits the weights (8 bytes an element, about
 // 230 us of a block at hidden 2560, SwiGLU 6912) costs more than it saves.
-// Whole fp32 block, library GEMMs against split ones: 512 rows 826 / 840 us,
-// 1000 rows 1410 / 1006 us, 2304 rows 2867 / 1482 us, 4600 rows 5530 / 2568 us;
-// at hidden 1024 and 512 rows 231 / 285 us.
-constexpr int kSplitMinRows = 768;
+// Whole fp32 block, library GEMMs against split ones: 144 rows 456 / 522 us,
+// 256 rows 559 / 546, 384 rows 708 / 621, 512 rows 826 / 671, 1000 rows 1399 / 916,
+// 2304 rows 2851 / 1378, 4600 rows 5525 / 2438; hidden 1024 and 512 rows 233 / 183.
+constexpr int kSplitMinRows = 320;
 
-bool use_split(const awa_dit_block* b, long long hd)
+// The kernel addresses its operands (at most 4 bytes a value) with 32-bit byte
+// offsets.
+bool addressable(const awa_dit_block* b, long long hd)
 {
     const awa_dit_block_desc& d = b->desc;
-    if (d.precision != AWA_COMPUTE_F32 || b->tokens[0] < kSplitMinRows)
-        return false;
-    // The kernel addresses planes with 32-bit byte offsets.
     const long long width = std::max({hd, static_cast<long long>(d.hidden), static_cast<long long>(d.mlp_hidden)});
     const long long rows = std::max({static_cast<long long>(b->tokens[0]), static_cast<long long>(b->tokens[1]), 3 * hd,
                                      static_cast<long long>(d.hidden), 2LL * d.mlp_hidden});
     return rows * groups_of(width) * 128 < (1LL << 32);
+}
+
+bool use_split(const awa_dit_block* b, long long hd)
+{
+    return b->desc.precision == AWA_COMPUTE_F32 && b->tokens[0] >= kSplitMinRows && addressable(b, hd);
+}
+
+// bf16 blocks run on the grouped GEMMs up to this many video rows, narrow ones
+// at any: beyond, the library's larger wave tiles gain more per MFMA than the
+// fused epilogues and the shared launch save. Whole bf16 block, library against
+// grouped GEMMs, hidden 2560: 81 rows (hidden 1024) 144 / 70 us, 256 rows
+// 234 / 185, 512 rows 270 / 243, 1000 rows 338 / 338, 2304 rows 532 / 496, 4600 rows
+// 826 / 824, 6400 rows 1136 / 1200, 9200 rows 1494 / 1520; hidden 1536, 9200 rows
+// 776 / 660; hidden 1024, 6400 rows 398 / 282.
+constexpr int kGroupedMaxRows = 5000;
+constexpr int kGroupedNarrow = 1536;
+
+// The kernel loads weights in 16-byte pieces.
+bool use_grouped(const awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2])
+{
+    if (b->split)
+        return true;
+    const awa_dit_block_desc& d = b->desc;
+    if (d.precision != AWA_COMPUTE_BF16 || (b->tokens[0] > kGroupedMaxRows && d.hidden > kGroupedNarrow) ||
+        !addressable(b, static_cast<long long>(d.heads) * d.head_dim))
+        return false;
+    for (const awa_dit_branch_weights* w : W)
+        for (const void* p : {w->qkv, w->proj_out, w->mlp_gate, w->mlp_in, w->mlp_out})
+            if (!aligned16(p))
+                return false;
+    return true;
 }
 
 int allocate_split(awa_dit_block* b, long long hd)
@@ -370,11 +405,6 @@ int allocate_split(awa_dit_block* b, long long hd)
     return AWA_OK;
 }
 
-bool aligned16(const void* p)
-{
-    return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
-}
-
 bool branch_weights_valid(const awa_dit_branch_weights* w, bool full)
 {
     if (!w || !w->qkv || !w->proj_out || !w->proj_out_bias || !w->norm_q || !w->norm_k)
@@ -398,15 +428,14 @@ int attention(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2], hip
     return awa::forward_fused(b->plan, &vq, &tq, &norm, &vo, &to, d.precision, stream, nullptr);
 }
 
-// One GEMM step of both branches on split operands: the weights are split,
-// then one launch runs the video and (text_rows > 0) the text GEMM. The
-// activations' planes are in place. in2: a second weight of the same size
-// whose rows follow the first's (SwiGLU).
-int split_gemm(awa_dit_block* b, const float* const (&w)[2], const float* const (&w2)[2], int n, int k, int text_rows,
-               awa::GemmLaunch& g, hipStream_t stream)
+// One GEMM step of both branches, the video and (text_rows > 0) the text GEMM
+// in one launch of csrc/dit_gemm.hip: A is ws[buf] (bf16) or the activations'
+// planes (split, where the weights are split first). w2: a second weight of
+// the same size for the other half of the n columns (SwiGLU).
+int gemm_step(awa_dit_block* b, int buf, const void* const (&w)[2], const void* const (&w2)[2], int n, int k,
+              int text_rows, awa::GemmLaunch& g, hipStream_t stream)
 {
     const int groups = groups_of(k);
-    const size_t pitch = static_cast<size_t>(groups) * 128;
     awa::SplitLaunch s{};
     s.width = k;
     s.groups = groups;
@@ -416,27 +445,43 @@ int split_gemm(awa_dit_block* b, const float* const (&w)[2], const float* const 
         q.m = br == 0 ? b->tokens[0] : text_rows;
         if (q.m <= 0)
             continue;
+        q.n = n;
+        if (!b->split)
+        {
+            q.a = b->ws[br][buf];
+            q.w = w[br];
+            q.w2 = w2[br];
+            q.lda = q.ldw = static_cast<uint32_t>(k) * 2;
+            q.stages = (k + 63) / 64;
+            q.last_bytes = static_cast<uint32_t>(k - (q.stages - 1) * 64) * 2;
+            continue;
+        }
+        const size_t pitch = static_cast<size_t>(groups) * 128;
         const int first = w2[br] ? n / 2 : n;
         char* planes = static_cast<char*>(b->planes[br][1]);
-        s.part[2 * br] = {w[br], planes, b->shifts[br][1], first};
+        s.part[2 * br] = {static_cast<const float*>(w[br]), planes, b->shifts[br][1], first};
         if (w2[br])
-            s.part[2 * br + 1] = {w2[br], planes + pitch * first, b->shifts[br][1] + first, n - first};
+            s.part[2 * br + 1] = {static_cast<const float*>(w2[br]), planes + pitch * first, b->shifts[br][1] + first,
+                                  n - first};
         q.a = b->planes[br][0];
         q.w = planes;
+        q.w2 = planes + pitch * first;
         q.meta_a = b->shifts[br][0];
         q.meta_w = b->shifts[br][1];
         q.lda = q.ldw = static_cast<uint32_t>(pitch);
-        q.n = n;
-        q.groups = groups;
+        q.stages = groups;
     }
-    DIT_HIP(awa::launch_split_rows(s, stream), "split_rows launch");
-    DIT_HIP(awa::launch_split_gemm(g, stream), "split GEMM launch");
+    if (b->split)
+        DIT_HIP(awa::launch_split_rows(s, stream), "split_rows launch");
+    DIT_HIP(awa::launch_gemm(g, b->split, stream), "GEMM launch");
     return AWA_OK;
 }
 
-// Splits activations of both branches into their planes.
+// fp32: splits activations of both branches into their planes.
 int split_activations(awa_dit_block* b, int buf, int width, int text_rows, hipStream_t stream)
 {
+    if (!b->split)
+        return AWA_OK;
     awa::SplitLaunch s{};
     s.width = width;
     s.groups = groups_of(width);
@@ -447,32 +492,32 @@ int split_activations(awa_dit_block* b, int buf, int width, int text_rows, hipSt
     return AWA_OK;
 }
 
-// The block on split fp32 GEMMs (csrc/dit_gemm.hip): the same steps, the video
-// and text GEMM of a step in one launch, the bias, gate, residual and SwiGLU in
-// the GEMMs' epilogues and the norm straight into fp16 planes.
-int forward_split(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2], const void* const (&in)[2],
-                  const void* emb, void* const (&out)[2], hipStream_t stream)
+// The block on the GEMMs of csrc/dit_gemm.hip: the same steps, the video and
+// text GEMM of a step in one launch, the bias, gate, residual and SwiGLU in
+// the GEMMs' epilogues and (fp32) the norm straight into fp16 planes.
+int forward_grouped(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2], const void* const (&in)[2],
+                    const void* emb, void* const (&out)[2], hipStream_t stream)
 {
     const awa_dit_block_desc& d = b->desc;
     const bool last = d.last_layer != 0;
     const int hidden = d.hidden, hd = d.heads * d.head_dim, mh = d.mlp_hidden;
     const int text = b->tokens[1];
     int rc;
-    auto weight = [](const void* p) { return static_cast<const float*>(p); };
-    const float* const none[2] = {nullptr, nullptr};
+    const void* const none[2] = {nullptr, nullptr};
     auto norm = [&](int br, const void* x, int shift_row, bool modulate) {
         awa::RowNormModulate nm{};
         nm.in = x;
-        nm.in_elemsize = 4;
+        nm.in_elemsize = b->es;
         nm.in_stride = hidden;
-        nm.out = b->planes[br][0];
-        nm.out_elemsize = 4;
+        nm.out = b->split ? b->planes[br][0] : b->ws[br][kNorm];
+        nm.out_elemsize = b->es;
+        nm.out_stride = hidden;
         nm.rows = b->tokens[br];
         nm.width = hidden;
         nm.eps = d.norm_eps;
         nm.shift = modulate ? b->ada[br] + static_cast<size_t>(shift_row) * hidden : nullptr;
         nm.scale = modulate ? b->ada[br] + static_cast<size_t>(shift_row + 1) * hidden : nullptr;
-        nm.meta = b->shifts[br][0];
+        nm.meta = b->split ? b->shifts[br][0] : nullptr;
         nm.groups = groups_of(hidden);
         return awa::launch_rmsnorm_modulate(nm, stream);
     };
@@ -481,7 +526,7 @@ int forward_split(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2],
     {
         const bool modulate = br == 0 || !last;
         if (modulate)
-            DIT_HIP(awa::launch_ada_prepare(emb, 4, W[br]->ada, b->ada[br], hidden, stream), "ada_prepare launch");
+            DIT_HIP(awa::launch_ada_prepare(emb, b->es, W[br]->ada, b->ada[br], hidden, stream), "ada_prepare launch");
         DIT_HIP(norm(br, in[br], 0, modulate), "rmsnorm_modulate launch");
     }
     {
@@ -492,8 +537,8 @@ int forward_split(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2],
             g.problem[br].out = b->ws[br][kQkv];
             g.problem[br].ldo = 3LL * hd;
         }
-        const float* const w[2] = {weight(W[0]->qkv), weight(W[1]->qkv)};
-        if ((rc = split_gemm(b, w, none, 3 * hd, hidden, text, g, stream)) != AWA_OK)
+        const void* const w[2] = {W[0]->qkv, W[1]->qkv};
+        if ((rc = gemm_step(b, kNorm, w, none, 3 * hd, hidden, text, g, stream)) != AWA_OK)
             return rc;
     }
     if ((rc = attention(b, W, stream)) != AWA_OK)
@@ -514,8 +559,8 @@ int forward_split(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2],
             q.residual = in[br];
             q.twice = !full;
         }
-        const float* const w[2] = {weight(W[0]->proj_out), weight(W[1]->proj_out)};
-        if ((rc = split_gemm(b, w, none, hidden, hd, text, g, stream)) != AWA_OK)
+        const void* const w[2] = {W[0]->proj_out, W[1]->proj_out};
+        if ((rc = gemm_step(b, kAtt, w, none, hidden, hd, text, g, stream)) != AWA_OK)
             return rc;
     }
     const int mlp_text = last ? 0 : text;
@@ -529,9 +574,9 @@ int forward_split(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2],
             g.problem[br].out = b->ws[br][kHidden];
             g.problem[br].ldo = mh;
         }
-        const float* const w[2] = {weight(W[0]->mlp_gate), weight(W[1]->mlp_gate)};
-        const float* const w2[2] = {weight(W[0]->mlp_in), weight(W[1]->mlp_in)};
-        if ((rc = split_gemm(b, w, w2, 2 * mh, hidden, mlp_text, g, stream)) != AWA_OK)
+        const void* const w[2] = {W[0]->mlp_gate, W[1]->mlp_gate};
+        const void* const w2[2] = {W[0]->mlp_in, W[1]->mlp_in};
+        if ((rc = gemm_step(b, kNorm, w, w2, 2 * mh, hidden, mlp_text, g, stream)) != AWA_OK)
             return rc;
     }
     if ((rc = split_activations(b, kHidden, mh, mlp_text, stream)) != AWA_OK)
@@ -546,8 +591,8 @@ int forward_split(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2],
         q.gate = b->ada[br] + static_cast<size_t>(5) * hidden;
         q.residual = b->ws[br][kResid];
     }
-    const float* const w[2] = {weight(W[0]->mlp_out), weight(W[1]->mlp_out)};
-    return split_gemm(b, w, none, hidden, mh, mlp_text, g, stream);
+    const void* const w[2] = {W[0]->mlp_out, W[1]->mlp_out};
+    return gemm_step(b, kHidden, w, none, hidden, mh, mlp_text, g, stream);
 }
 
 } // namespace
@@ -653,8 +698,8 @@ int awa_dit_block_forward(awa_dit_block* b, const awa_dit_branch_weights* video_
     const awa_dit_branch_weights* const W[2] = {video_w, text_w};
     const void* const in[2] = {video, text};
     void* const out[2] = {video_out, text_out};
-    if (b->split)
-        return forward_split(b, W, in, emb, out, stream);
+    if (use_grouped(b, W))
+        return forward_grouped(b, W, in, emb, out, stream);
     int rc;
 
     // Attention half: Ada vectors, norm + Ada in, QKV projection.
