@@ -11,10 +11,18 @@ namespace awa
 {
 
 // ada[r][c] = emb[c][r / 3][r % 3] + learned[r][c] for the 6 rows (attn
-// shift, scale, gate, mlp shift, scale, gate) of one branch: the Ada vectors
-// the row kernels below read.
-hipError_t launch_ada_prepare(const void* emb, int emb_elemsize, const float* learned, float* ada, int width,
-                              hipStream_t stream);
+// shift, scale, gate, mlp shift, scale, gate) of each branch (learned = null:
+// none): the Ada vectors the row kernels below read.
+struct AdaPrepare
+{
+    const void* emb;
+    int emb_elemsize;
+    const float* learned[2];
+    float* ada[2];
+    int width;
+};
+
+hipError_t launch_ada_prepare(const AdaPrepare& p, hipStream_t stream);
 
 // out = rmsnorm(in) * scale + shift, per row of `width`; scale = shift = null
 // skips the modulation.
@@ -34,6 +42,12 @@ struct RowNormModulate
     // a row) and meta their shifts instead of the rows themselves.
     int* meta = nullptr;
     int groups = 0;
+};
+
+// Both branches' rows (rows = 0: none), both with meta or both without.
+struct RowNormPair
+{
+    RowNormModulate branch[2];
 };
 
 // out = (h + bias) * gate + residual (bias may be null; gate = null takes it as 1).
@@ -122,7 +136,7 @@ struct GemmLaunch
 hipError_t launch_split_rows(const SplitLaunch& p, hipStream_t stream);
 hipError_t launch_gemm(const GemmLaunch& p, bool split, hipStream_t stream);
 
-hipError_t launch_rmsnorm_modulate(const RowNormModulate& p, hipStream_t stream);
+hipError_t launch_rmsnorm_modulate(const RowNormPair& pair, hipStream_t stream);
 hipError_t launch_gate_residual(const GateResidual& p, hipStream_t stream);
 hipError_t launch_swiglu(const SwiGlu& p, hipStream_t stream);
 hipError_t launch_double(const void* in, int in_elemsize, long long in_stride, void* out, int out_elemsize,

@@ -110,16 +110,16 @@ __device__ __forceinline__ void load8f(const float* p, int i, float (&v)[8])
     v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
 }
 
-// ada[r][c] = emb[c * 6 + r] + learned[r][c] (r = 3 * layer + k).
-__global__ __launch_bounds__(kRowThreads) void ada_prepare_kernel(const void* emb, int emb_elemsize,
-                                                                  const float* learned, float* ada, int width)
+// ada[r][c] = emb[c * 6 + r] + learned[r][c] of branch blockIdx.y.
+__global__ __launch_bounds__(kRowThreads) void ada_prepare_kernel(const AdaPrepare p)
 {
     const int i = blockIdx.x * kRowThreads + threadIdx.x;
-    if (i >= 6 * width)
+    const int br = blockIdx.y;
+    if (i >= 6 * p.width || !p.learned[br])
         return;
-    const int r = i / width;
-    const int c = i - r * width;
-    ada[i] = load_act(emb, static_cast<long long>(c) * 6 + r, emb_elemsize) + learned[i];
+    const int r = i / p.width;
+    const int c = i - r * p.width;
+    p.ada[br][i] = load_act(p.emb, static_cast<long long>(c) * 6 + r, p.emb_elemsize) + p.learned[br][i];
 }
 
 constexpr int kRowChunks = 4; // chunks of 8 a thread keeps in registers (rows up to 8192 wide)
@@ -152,12 +152,16 @@ __device__ __forceinline__ void block_max(uint32_t& max, int& flags, uint32_t* r
 // y = rmsnorm(x) * (scale_a + scale_b) + (shift_a + shift_b), one workgroup
 // per row; the row stays in registers between the two passes. PLANES: y goes
 // out as fp16 planes for a split GEMM (its scan and a pass over y saved).
+// The text rows' workgroups follow the video rows' (a launch of their own
+// took 5 us beside the video's 10 at 2304 rows).
 template <bool PLANES>
-__global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const RowNormModulate p)
+__global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const RowNormPair pair)
 {
+    const int video_rows = pair.branch[0].rows;
+    const RowNormModulate& p = pair.branch[static_cast<int>(blockIdx.x) < video_rows ? 0 : 1];
     __shared__ float red[4];
     __shared__ uint32_t red_max[8];
-    const long long row = blockIdx.x;
+    const long long row = static_cast<int>(blockIdx.x) < video_rows ? blockIdx.x : blockIdx.x - video_rows;
     const int chunks = p.width / 8;
     const long long base_in = row * p.in_stride;
     float v[kRowChunks][8];
@@ -303,26 +307,36 @@ int elementwise_grid(long long n)
 
 } // namespace
 
-hipError_t launch_ada_prepare(const void* emb, int emb_elemsize, const float* learned, float* ada, int width,
-                              hipStream_t stream)
+hipError_t launch_ada_prepare(const AdaPrepare& p, hipStream_t stream)
 {
-    if (width <= 0)
+    if (p.width <= 0)
         return hipSuccess;
-    hipLaunchKernelGGL(ada_prepare_kernel, dim3((6 * width + kRowThreads - 1) / kRowThreads), dim3(kRowThreads), 0,
-                       stream, emb, emb_elemsize, learned, ada, width);
+    hipLaunchKernelGGL(ada_prepare_kernel, dim3((6 * p.width + kRowThreads - 1) / kRowThreads, 2), dim3(kRowThreads),
+                       0, stream, p);
     return hipGetLastError();
 }
 
-hipError_t launch_rmsnorm_modulate(const RowNormModulate& p, hipStream_t stream)
+hipError_t launch_rmsnorm_modulate(const RowNormPair& pair, hipStream_t stream)
 {
-    if (p.rows <= 0)
+    long long rows = 0;
+    bool planes = false;
+    for (const RowNormModulate& p : pair.branch)
+    {
+        if (p.rows <= 0)
+            continue;
+        if (p.width % 8 || p.width > 8 * kRowChunks * kRowThreads || p.in_stride % 8 || p.out_stride % 8)
+            return hipErrorInvalidValue;
+        rows += p.rows;
+        planes = p.meta != nullptr;
+    }
+    if (rows <= 0)
         return hipSuccess;
-    if (p.width % 8 || p.width > 8 * kRowChunks * kRowThreads || p.in_stride % 8 || p.out_stride % 8)
-        return hipErrorInvalidValue;
-    if (p.meta)
-        hipLaunchKernelGGL(rmsnorm_modulate_kernel<true>, dim3(p.rows), dim3(kRowThreads), 0, stream, p);
+    if (planes)
+        hipLaunchKernelGGL(rmsnorm_modulate_kernel<true>, dim3(static_cast<unsigned>(rows)), dim3(kRowThreads), 0,
+                           stream, pair);
     else
-        hipLaunchKernelGGL(rmsnorm_modulate_kernel<false>, dim3(p.rows), dim3(kRowThreads), 0, stream, p);
+        hipLaunchKernelGGL(rmsnorm_modulate_kernel<false>, dim3(static_cast<unsigned>(rows)), dim3(kRowThreads), 0,
+                           stream, pair);
     return hipGetLastError();
 }
 

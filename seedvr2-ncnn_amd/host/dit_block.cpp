@@ -416,6 +416,15 @@ bool branch_weights_valid(const awa_dit_branch_weights* w, bool full)
     return true;
 }
 
+// Both branches' Ada vectors (the last block modulates video only).
+hipError_t ada_prepare(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2], const void* emb,
+                       hipStream_t stream)
+{
+    awa::AdaPrepare p{emb, b->es, {W[0]->ada, b->desc.last_layer ? nullptr : W[1]->ada}, {b->ada[0], b->ada[1]},
+                      b->desc.hidden};
+    return awa::launch_ada_prepare(p, stream);
+}
+
 // AWA with the q/k RMSNorm fused into its gather.
 int attention(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2], hipStream_t stream)
 {
@@ -504,31 +513,32 @@ int forward_grouped(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2
     const int text = b->tokens[1];
     int rc;
     const void* const none[2] = {nullptr, nullptr};
-    auto norm = [&](int br, const void* x, int shift_row, bool modulate) {
-        awa::RowNormModulate nm{};
-        nm.in = x;
-        nm.in_elemsize = b->es;
-        nm.in_stride = hidden;
-        nm.out = b->split ? b->planes[br][0] : b->ws[br][kNorm];
-        nm.out_elemsize = b->es;
-        nm.out_stride = hidden;
-        nm.rows = b->tokens[br];
-        nm.width = hidden;
-        nm.eps = d.norm_eps;
-        nm.shift = modulate ? b->ada[br] + static_cast<size_t>(shift_row) * hidden : nullptr;
-        nm.scale = modulate ? b->ada[br] + static_cast<size_t>(shift_row + 1) * hidden : nullptr;
-        nm.meta = b->split ? b->shifts[br][0] : nullptr;
-        nm.groups = groups_of(hidden);
-        return awa::launch_rmsnorm_modulate(nm, stream);
+    // Norm + Ada "in" of rows x: shift and scale rows shift_row, shift_row + 1.
+    auto norm = [&](const void* const (&x)[2], int shift_row, int text_rows, bool modulate_text) {
+        awa::RowNormPair pair{};
+        for (int br = 0; br < 2; br++)
+        {
+            const bool modulate = br == 0 || modulate_text;
+            awa::RowNormModulate& nm = pair.branch[br];
+            nm.in = x[br];
+            nm.in_elemsize = b->es;
+            nm.in_stride = hidden;
+            nm.out = b->split ? b->planes[br][0] : b->ws[br][kNorm];
+            nm.out_elemsize = b->es;
+            nm.out_stride = hidden;
+            nm.rows = br == 0 ? b->tokens[0] : text_rows;
+            nm.width = hidden;
+            nm.eps = d.norm_eps;
+            nm.shift = modulate ? b->ada[br] + static_cast<size_t>(shift_row) * hidden : nullptr;
+            nm.scale = modulate ? b->ada[br] + static_cast<size_t>(shift_row + 1) * hidden : nullptr;
+            nm.meta = b->split ? b->shifts[br][0] : nullptr;
+            nm.groups = groups_of(hidden);
+        }
+        return awa::launch_rmsnorm_modulate(pair, stream);
     };
 
-    for (int br = 0; br < 2; br++)
-    {
-        const bool modulate = br == 0 || !last;
-        if (modulate)
-            DIT_HIP(awa::launch_ada_prepare(emb, b->es, W[br]->ada, b->ada[br], hidden, stream), "ada_prepare launch");
-        DIT_HIP(norm(br, in[br], 0, modulate), "rmsnorm_modulate launch");
-    }
+    DIT_HIP(ada_prepare(b, W, emb, stream), "ada_prepare launch");
+    DIT_HIP(norm(in, 0, text, !last), "rmsnorm_modulate launch");
     {
         awa::GemmLaunch g{};
         g.epilogue = awa::kGemmStore;
@@ -564,8 +574,8 @@ int forward_grouped(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2
             return rc;
     }
     const int mlp_text = last ? 0 : text;
-    for (int br = 0; br < (last ? 1 : 2); br++)
-        DIT_HIP(norm(br, b->ws[br][kResid], 3, true), "rmsnorm_modulate launch");
+    const void* const resid[2] = {b->ws[0][kResid], b->ws[1][kResid]};
+    DIT_HIP(norm(resid, 3, mlp_text, true), "rmsnorm_modulate launch");
     {
         awa::GemmLaunch g{};
         g.epilogue = awa::kGemmSwiGlu;
@@ -703,13 +713,13 @@ int awa_dit_block_forward(awa_dit_block* b, const awa_dit_branch_weights* video_
     int rc;
 
     // Attention half: Ada vectors, norm + Ada in, QKV projection.
+    DIT_HIP(ada_prepare(b, W, emb, stream), "ada_prepare launch");
     for (int br = 0; br < 2; br++)
     {
         const int M = b->tokens[br];
         const bool modulate = br == 0 || !last;
-        if (modulate)
-            DIT_HIP(awa::launch_ada_prepare(emb, es, W[br]->ada, b->ada[br], hidden, stream), "ada_prepare launch");
-        awa::RowNormModulate nm{};
+        awa::RowNormPair rows{};
+        awa::RowNormModulate& nm = rows.branch[0];
         nm.in = in[br];
         nm.in_elemsize = es;
         nm.in_stride = hidden;
@@ -721,7 +731,7 @@ int awa_dit_block_forward(awa_dit_block* b, const awa_dit_branch_weights* video_
         nm.eps = d.norm_eps;
         nm.shift = modulate ? b->ada[br] + 0 * hidden : nullptr;
         nm.scale = modulate ? b->ada[br] + 1 * hidden : nullptr;
-        DIT_HIP(awa::launch_rmsnorm_modulate(nm, stream), "rmsnorm_modulate launch");
+        DIT_HIP(awa::launch_rmsnorm_modulate(rows, stream), "rmsnorm_modulate launch");
         if ((rc = gemm(b, b->ws[br][kNorm], hidden, W[br]->qkv, b->ws[br][kQkv], 3LL * hd, M, 3 * hd, hidden,
                        stream)) != AWA_OK)
             return rc;
@@ -758,7 +768,8 @@ int awa_dit_block_forward(awa_dit_block* b, const awa_dit_branch_weights* video_
             continue;
         }
         // MLP half: norm + Ada in (mlp), SwiGLU, output projection, gate + residual.
-        awa::RowNormModulate nm{};
+        awa::RowNormPair rows{};
+        awa::RowNormModulate& nm = rows.branch[0];
         nm.in = b->ws[br][kResid];
         nm.in_elemsize = es;
         nm.in_stride = hidden;
@@ -770,7 +781,7 @@ int awa_dit_block_forward(awa_dit_block* b, const awa_dit_branch_weights* video_
         nm.eps = d.norm_eps;
         nm.shift = b->ada[br] + 3 * hidden;
         nm.scale = b->ada[br] + 4 * hidden;
-        DIT_HIP(awa::launch_rmsnorm_modulate(nm, stream), "rmsnorm_modulate launch");
+        DIT_HIP(awa::launch_rmsnorm_modulate(rows, stream), "rmsnorm_modulate launch");
         char* pair = static_cast<char*>(b->ws[br][kPair]);
         // The two input projections fill the halves of one [M][2 mh] buffer.
         // Weights stored back to back ([mh][hidden] gate, then in) are one
