@@ -439,8 +439,9 @@ int attention(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2], hip
 
 // One GEMM step of both branches, the video and (text_rows > 0) the text GEMM
 // in one launch of csrc/dit_gemm.hip: A is ws[buf] (bf16) or the activations'
-// planes (split, where the weights are split first). w2: a second weight of
-// the same size for the other half of the n columns (SwiGLU).
+// planes (split, where the weights are split first, and in the same launch the
+// activations in ws[buf] unless the norm has left their planes). w2: a second
+// weight of the same size for the other half of the n columns (SwiGLU).
 int gemm_step(awa_dit_block* b, int buf, const void* const (&w)[2], const void* const (&w2)[2], int n, int k,
               int text_rows, awa::GemmLaunch& g, hipStream_t stream)
 {
@@ -465,6 +466,8 @@ int gemm_step(awa_dit_block* b, int buf, const void* const (&w)[2], const void* 
             q.last_bytes = static_cast<uint32_t>(k - (q.stages - 1) * 64) * 2;
             continue;
         }
+        if (buf != kNorm)
+            s.part[2 * br + 1] = {static_cast<const float*>(b->ws[br][buf]), b->planes[br][0], b->shifts[br][0], q.m};
         const size_t pitch = static_cast<size_t>(groups) * 128;
         const int first = w2[br] ? n / 2 : n;
         char* planes = static_cast<char*>(b->planes[br][1]);
@@ -483,21 +486,6 @@ int gemm_step(awa_dit_block* b, int buf, const void* const (&w)[2], const void* 
     if (b->split)
         DIT_HIP(awa::launch_split_rows(s, stream), "split_rows launch");
     DIT_HIP(awa::launch_gemm(g, b->split, stream), "GEMM launch");
-    return AWA_OK;
-}
-
-// fp32: splits activations of both branches into their planes.
-int split_activations(awa_dit_block* b, int buf, int width, int text_rows, hipStream_t stream)
-{
-    if (!b->split)
-        return AWA_OK;
-    awa::SplitLaunch s{};
-    s.width = width;
-    s.groups = groups_of(width);
-    for (int br = 0; br < 2; br++)
-        s.part[br] = {static_cast<const float*>(b->ws[br][buf]), b->planes[br][0], b->shifts[br][0],
-                      br == 0 ? b->tokens[0] : text_rows};
-    DIT_HIP(awa::launch_split_rows(s, stream), "split_rows launch");
     return AWA_OK;
 }
 
@@ -553,8 +541,6 @@ int forward_grouped(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2
     }
     if ((rc = attention(b, W, stream)) != AWA_OK)
         return rc;
-    if ((rc = split_activations(b, kAtt, hd, text, stream)) != AWA_OK)
-        return rc;
     {
         awa::GemmLaunch g{};
         g.epilogue = awa::kGemmGate;
@@ -589,8 +575,6 @@ int forward_grouped(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2
         if ((rc = gemm_step(b, kNorm, w, w2, 2 * mh, hidden, mlp_text, g, stream)) != AWA_OK)
             return rc;
     }
-    if ((rc = split_activations(b, kHidden, mh, mlp_text, stream)) != AWA_OK)
-        return rc;
     awa::GemmLaunch g{};
     g.epilogue = awa::kGemmGate;
     for (int br = 0; br < 2; br++)

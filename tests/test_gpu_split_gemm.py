@@ -129,3 +129,20 @@ def test_split_block_infinite_and_nan_weights(gpu):
         for col in (37, 200):
             assert np.array_equal(a[:, col].astype(np.float64), b[:, col])
         assert off(a[:, keep], c[:, keep]) <= 1e-5
+
+
+def test_split_block_infinite_hidden_value(gpu):
+    """An infinite weight of mlp_in makes one hidden value of every row
+    infinite (the SwiGLU epilogue), and with it every output, with the sign
+    that value and its mlp_out weight give."""
+    print("case split block infinite hidden value", flush=True)
+    grid, heads, hidden, mlp = (3, 16, 16), 2, 256, 384
+    g, video, txt, emb, wv, wt = inputs(8, grid, 8, heads, hidden, mlp)
+    for w in (wv, wt):
+        w.mlp_in[5, 7] = np.inf
+    got = run(g, video, txt, emb, wv, wt, heads, hidden, mlp)
+    with np.errstate(invalid="ignore"):
+        ref = O.dit_block(g, video, txt, emb, wv, wt, heads, HEAD_DIM, EPS, False)
+    for a, b in zip(got, ref):
+        assert np.all(np.isinf(b))
+        assert np.array_equal(a.astype(np.float64), b)
