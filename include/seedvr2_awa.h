@@ -317,18 +317,24 @@ int awa_stack_block_flops(const awa_stack* stack, double* flops);
  * precision AWA_COMPUTE_F32: fp32 activations, GEMM weights and GEMMs (the
  * FP32 prefix blocks); AWA_COMPUTE_BF16: bf16 activations and GEMM weights,
  * fp32 accumulation and arithmetic (the BF16 blocks, dit_stack.cpp:519,
- * :550). The GEMMs are library GEMMs (hipBLASLt). A block or stack object is
- * used by one thread at a time (it caches GEMM descriptors on first use). The
- * first GEMM of each shape in the process times hipBLASLt's candidate
- * algorithms on the caller's operands and stream, waiting for the stream once
- * (not under graph capture, where the heuristic's first is taken for that
- * call); its choice then holds for every block and stack object of the
- * process, so equal shapes give equal bits within a process. Timing noise can
- * still pick a different algorithm in another process, and results then differ
- * in the last bits (the fp32 and bf16 tolerances hold either way). With the
- * environment variable SEEDVR2_GEMM_HEURISTIC=1 the heuristic's first
- * algorithm is taken for every shape, without timing: the same choice in every
- * process on the same device and library version. */
+ * :550). The GEMMs run on the build's own kernel, video and text rows in one
+ * launch: bf16 MFMA, or for fp32 blocks each operand row as two fp16 planes (22
+ * bits and the signs, or 2^-40 of the row's largest value), three fp16 MFMAs a
+ * product with fp32 accumulation, no further from the exact product than fp32
+ * MFMAs are. NaN and infinities of fp32 operands reach the outputs they would
+ * reach in fp32. Equal shapes give equal bits in every process.
+ * Library GEMMs (hipBLASLt) serve fp32 blocks of fewer than 320 video rows, bf16
+ * blocks of more than 5000 video rows at hidden > 1536, operands past 4 GiB
+ * and bf16 weights off 16-byte addresses. There the first GEMM of each shape in
+ * the process times hipBLASLt's candidate algorithms on the caller's operands
+ * and stream, waiting for the stream once (not under graph capture, where the
+ * heuristic's first is taken for that call); its choice then holds for every
+ * block and stack object of the process, and another process may choose
+ * otherwise (last bits). With the environment variable
+ * SEEDVR2_GEMM_HEURISTIC=1 the heuristic's first algorithm is taken for every
+ * shape, without timing. An fp32 block on split GEMMs keeps planes of its largest
+ * weight, 4 bytes a value and branch. A block or stack object is used by one
+ * thread at a time. */
 typedef struct awa_dit_block_desc {
     int source_t, source_h, source_w;    /* token grid */
     int windows_t, windows_h, windows_w; /* window counts (params 3/4/5) */
@@ -353,7 +359,7 @@ typedef struct awa_dit_branch_weights {
     const float* proj_out_bias; /* [hidden], 16-byte aligned */
     const void* mlp_gate;       /* [mlp_hidden][hidden] (proj_in_gate) */
     const void* mlp_in;         /* [mlp_hidden][hidden] (proj_in); stored right after mlp_gate, the two
-                                   run as one GEMM of width 2 * mlp_hidden */
+                                   run as one library GEMM of width 2 * mlp_hidden */
     const void* mlp_out;        /* [hidden][mlp_hidden] (proj_out) */
     const float* norm_q;        /* [head_dim], 16-byte aligned */
     const float* norm_k;        /* [head_dim], 16-byte aligned */
