@@ -319,10 +319,13 @@ int awa_stack_block_flops(const awa_stack* stack, double* flops);
  * fp32 accumulation and arithmetic (the BF16 blocks, dit_stack.cpp:519,
  * :550). The GEMMs run on the build's own kernel, video and text rows in one
  * launch: bf16 MFMA, or for fp32 blocks each operand row as two fp16 planes (22
- * bits and the signs, or 2^-40 of the row's largest value), three fp16 MFMAs a
- * product with fp32 accumulation, no further from the exact product than fp32
- * MFMAs are. NaN and infinities of fp32 operands reach the outputs they would
- * reach in fp32. Equal shapes give equal bits in every process.
+ * bits and the sign of a value), three fp16 MFMAs a product with fp32
+ * accumulation. A value below 2^-18 of its row's largest keeps fewer bits there,
+ * so each output to which such values could contribute more than 2^-22 of itself
+ * is computed from the fp32 operands instead, and so is every output of a row
+ * with a NaN or an infinity: those reach the outputs they reach in fp32. A block
+ * whose data mark many outputs takes longer, up to about twice the time of
+ * the library's fp32 GEMMs. Equal shapes give equal bits in every process.
  * Library GEMMs (hipBLASLt) serve fp32 blocks of fewer than 320 video rows, bf16
  * blocks of more than 5000 video rows at hidden > 1536, operands past 4 GiB
  * and bf16 weights off 16-byte addresses. There the first GEMM of each shape in

@@ -5,12 +5,19 @@
 // fp32 operands are split. A row x (of A or of W) is stored as x 2^s = hi + lo
 // with s the row's exponent shift (its largest finite value lies in
 // [2^14, 2^15)), hi the value rounded to fp16 and lo the rest rounded to fp16:
-// 22 bits and the signs, or 2^-40 of the row's largest value where that is
-// coarser. The product is hi hi + hi lo + lo hi on v_mfma_f32_32x32x16_f16
-// with fp32 accumulation (the dropped lo lo weighs 2^-24 of a product), three
-// fp16 MFMAs in place of one fp32 product at 1/16 of their rate. Off the
-// 64-bit product by 5.7e-7 (relative 2-norm, N(0, 1) by N(0, 0.02), K = 2560)
-// where fp32 MFMAs are off by 9.0e-7.
+// 2^-22 of a value down to 2^-18 of the row's largest. The product is hi hi +
+// hi lo + lo hi on v_mfma_f32_32x32x16_f16 with fp32 accumulation (the dropped
+// lo lo weighs at most 2^-22 of a product), three fp16 MFMAs in place of one
+// fp32 product at 1/16 of their rate. Off the 64-bit product by 5.7e-7 (relative
+// 2-norm, N(0, 1) by N(0, 0.02), K = 2560) where fp32 MFMAs are off by 9.0e-7.
+// Smaller values lose bits, down to all of them: each row's meta holds what its
+// planes dropped, and an output of which that could be more than 2^-22 is
+// computed from the fp32 rows instead (finish_marked), as is every output of a
+// row with a NaN or an infinity. A few in 1e6 outputs of a SwiGLU's second GEMM,
+// none of N(0, 1) rows: the 33-frame fp32 block takes 1380 us with the check and
+// 1357 without. What the marked ones cost there, beside 2890 us of the library's
+// fp32 GEMMs: an infinite weight 2060 us, four hidden features 2^20 larger than the
+// rest 2970, every output of two GEMMs marked 5220.
 //
 // What bounds the stage loop is the matrix core and, next, what feeds it: LDS
 // (a 256 x 256 bf16 stage is 2048 MFMA cycles a SIMD and as many of LDS reads
@@ -119,49 +126,234 @@ __device__ __forceinline__ void store8(void* p, size_t i, const float (&v)[8])
     }
 }
 
-// One product of split rows of which one is not finite, from the planes in
-// fp32: an infinity stays one where the split products would give NaN.
-__device__ float dot_planes(const GemmProblem& g, const void* weight, int row, int wrow, int ma, int mw)
+// A row of a split GEMM's operand: its planes where they keep every value's 22
+// bits, else the fp32 row.
+struct OperandRow
 {
-    if ((ma | mw) & kRowNan)
-        return __uint_as_float(0x7fc00000u);
-    const char* a = static_cast<const char*>(g.a) + static_cast<size_t>(row) * g.lda;
-    const char* w = static_cast<const char*>(weight) + static_cast<size_t>(wrow) * g.ldw;
-    float sum = 0.f;
-    for (int t = 0; t < g.stages; t++)
-    {
-        const _Float16* pa = reinterpret_cast<const _Float16*>(a + static_cast<size_t>(t) * kStageBytes);
-        const _Float16* pw = reinterpret_cast<const _Float16*>(w + static_cast<size_t>(t) * kStageBytes);
-        for (int k = 0; k < kGroup; k++)
-            sum = fmaf(static_cast<float>(pa[k]) + static_cast<float>(pa[k + kGroup]),
-                       static_cast<float>(pw[k]) + static_cast<float>(pw[k + kGroup]), sum);
-    }
-    return ldexpf(sum, -row_shift(ma) - row_shift(mw));
+    const char* at;
+    int shift;
+    bool full;
+};
+
+__device__ __forceinline__ OperandRow operand_row(const float* full, const void* planes, uint32_t pitch, int width,
+                                                  int row, const RowMeta& meta)
+{
+    if (meta.loss == 0.f)
+        return {static_cast<const char*>(planes) + static_cast<size_t>(row) * pitch, meta.shift, false};
+    return {reinterpret_cast<const char*>(full + static_cast<size_t>(row) * width), 0, true};
 }
 
-// The outputs of a wave's tile whose row or column holds a NaN or an infinity.
-template <int EPI>
-__device__ void finish_non_finite(const GemmProblem& g, int row0, int rows, int col0, int cols)
+__device__ __forceinline__ OperandRow operand_a(const GemmProblem& g, int row)
 {
-    const int width = EPI == kGemmSwiGlu ? g.n >> 1 : g.n;
-    for (int i = threadIdx.x & 63; i < rows * cols; i += 64)
+    return operand_row(g.full_a, g.a, g.lda, g.width, row, g.meta_a[row]);
+}
+
+// Row c of w, or of w2 (SwiGLU).
+__device__ __forceinline__ OperandRow operand_w(const GemmProblem& g, int c, bool second)
+{
+    return operand_row(second ? g.full_w2 : g.full_w, second ? g.w2 : g.w, g.ldw, g.width, c,
+                       g.meta_w[second ? (g.n >> 1) + c : c]);
+}
+
+// Eight values of a row as they lie in memory (fp32, or hi and lo), so that a
+// load is not waited for before they are used.
+struct Raw8
+{
+    uint4 x, y;
+};
+
+__device__ __forceinline__ Raw8 load_operand(const OperandRow& r, int k)
+{
+    typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(4)));
+    const char* at = r.at + (r.full ? 4 * k : k / kGroup * kStageBytes + k % kGroup * 2);
+    const uint4u x = *reinterpret_cast<const uint4u*>(at);
+    const uint4u y = *reinterpret_cast<const uint4u*>(at + (r.full ? 16 : 2 * kGroup));
+    return {__builtin_bit_cast(uint4, x), __builtin_bit_cast(uint4, y)};
+}
+
+__device__ __forceinline__ void operand_values(const OperandRow& r, const Raw8& raw, float (&v)[8])
+{
+    const half8 hi = __builtin_bit_cast(half8, raw.x), lo = __builtin_bit_cast(half8, raw.y);
+    const float full[8] = {__uint_as_float(raw.x.x), __uint_as_float(raw.x.y), __uint_as_float(raw.x.z),
+                           __uint_as_float(raw.x.w), __uint_as_float(raw.y.x), __uint_as_float(raw.y.y),
+                           __uint_as_float(raw.y.z), __uint_as_float(raw.y.w)};
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        v[e] = r.full ? full[e] : ldexpf(static_cast<float>(hi[e]) + static_cast<float>(lo[e]), -r.shift);
+}
+
+// One product of two rows, the lanes of a wave along K. Bound by latency: the
+// loads of kAhead steps are in flight together.
+__device__ __forceinline__ float row_product(const OperandRow& a, const OperandRow& w, int width)
+{
+    constexpr int kAhead = 4;
+    float sum = 0.f;
+#pragma unroll 1
+    for (int k = (threadIdx.x & 63) * 8; k < width; k += 512 * kAhead)
     {
-        const int row = row0 + i / cols, c = col0 + i % cols;
-        if (row >= g.m || c >= width)
-            continue;
-        const int ma = g.meta_a[row], mw = g.meta_w[c], mi = EPI == kGemmSwiGlu ? g.meta_w[width + c] : 0;
-        if (!((ma | mw | mi) & (kRowNan | kRowInf)))
-            continue;
-        float r = dot_planes(g, g.w, row, c, ma, mw);
-        if (EPI == kGemmSwiGlu)
-            r = silu_mul<false>(r, dot_planes(g, g.w2, row, c, ma, mi));
-        if (EPI == kGemmGate)
+        Raw8 x[kAhead], y[kAhead];
+#pragma unroll
+        for (int s = 0; s < kAhead; s++)
         {
-            r = (r + (g.bias ? g.bias[c] : 0.f)) * (g.gate ? g.gate[c] : 1.f) +
-                static_cast<const float*>(g.residual)[static_cast<size_t>(row) * g.ldr + c];
-            r = g.twice ? r + r : r;
+            // Past the end: the last eight again, not summed.
+            x[s] = load_operand(a, min(k + 512 * s, width - 8));
+            y[s] = load_operand(w, min(k + 512 * s, width - 8));
         }
-        static_cast<float*>(g.out)[static_cast<size_t>(row) * g.ldo + c] = r;
+#pragma unroll
+        for (int s = 0; s < kAhead; s++)
+        {
+            float u[8], v[8];
+            operand_values(a, x[s], u);
+            operand_values(w, y[s], v);
+            if (k + 512 * s < width)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    sum = fmaf(u[e], v[e], sum);
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+        sum += __shfl_xor(sum, off, 64);
+    return sum;
+}
+
+// The products of 32 by 32 rows on the fp32 matrix core (lane l holds row
+// l % 32 of both and, of every 32 values, the 16 at 16 (l / 32)); laid out as
+// the accumulators of run_tile. A step takes whole 128-byte lines of every row
+// (the rows of a CU's waves do not fit its L1, so a line read by halves comes
+// from L2 twice), and the next step's are loaded while the matrix core works.
+__device__ __forceinline__ f32x16 block_product(const OperandRow& a, const OperandRow& w, int width)
+{
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++)
+        acc[e] = 0.f;
+    const int first = ((threadIdx.x >> 5) & 1) * 16;
+    Raw8 x[2], y[2];
+    // Past the rows' end: the last eight values, which a step then takes as zeros.
+    auto load = [&](int k) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+        {
+            x[h] = load_operand(a, min(k + first + 8 * h, width - 8));
+            y[h] = load_operand(w, min(k + first + 8 * h, width - 8));
+        }
+    };
+    auto step = [&](int k, bool tail) {
+        const Raw8 p[2] = {x[0], x[1]}, q[2] = {y[0], y[1]};
+        if (!tail)
+            load(k + 32);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+        {
+            float u[8], v[8];
+            operand_values(a, p[h], u);
+            operand_values(w, q[h], v);
+            if (tail && k + first + 8 * h >= width)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    u[e] = v[e] = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(u[e], v[e], acc, 0, 0, 0);
+        }
+    };
+    load(0);
+    int k = 0;
+    for (; k + 32 < width; k += 32)
+        step(k, false);
+    step(k, true);
+    return acc;
+}
+
+// One output of a split GEMM from its product(s).
+template <int EPI>
+__device__ __forceinline__ void store_output(const GemmProblem& g, int row, int c, float y, float z)
+{
+    if (EPI == kGemmSwiGlu)
+        y = silu_mul<false>(y, z);
+    if (EPI == kGemmGate)
+    {
+        y = (y + (g.bias ? g.bias[c] : 0.f)) * (g.gate ? g.gate[c] : 1.f) +
+            static_cast<const float*>(g.residual)[static_cast<size_t>(row) * g.ldr + c];
+        y = g.twice ? y + y : y;
+    }
+    static_cast<float*>(g.out)[static_cast<size_t>(row) * g.ldo + c] = y;
+}
+
+// Up to this many marked outputs of 32 rows of a wave's tile are computed one
+// by one (about 6 us each at K = 6912), more of them by blocks of 32 x 32. One
+// marked column of all rows (an infinite weight) takes the 33-frame fp32 block
+// 2150 us one by one and 2540 by blocks.
+constexpr int kFewMarked = 32;
+
+// The marked outputs of a wave's tile (rows from row0, output columns from
+// col0), from the fp32 operands. Lane l's marks of 32 rows m: bit 8 s + e is
+// column 8 (i % kChunks) + e of row i / kChunks, i = l + 64 s (the epilogue's
+// order). Rare: values of one row that differ by more than 2^18 and carry the
+// output, infinities and NaN.
+template <int EPI, int MB, int NB>
+__device__ void finish_marked(const GemmProblem& g, const uint64_t* marks, int row0, int col0)
+{
+    constexpr bool kPair = EPI == kGemmSwiGlu;
+    constexpr int kBlockCols = kPair ? 16 : 32; // output columns of a 32-column block
+    constexpr int kChunks = NB * kBlockCols / 8, kSteps = kChunks / 2;
+    static_assert(kChunks % 2 == 0 && kSteps <= 8, "marks of a lane in 64 bits");
+    const int lane = threadIdx.x & 63;
+    const int width = kPair ? g.n >> 1 : g.n;
+#pragma unroll 1
+    for (int m = 0; m < MB; m++)
+    {
+        uint64_t mine = marks[m * 64 + lane];
+        int count = __popcll(mine);
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1)
+            count += __shfl_xor(count, off, 64);
+        if (count == 0)
+            continue;
+        if (count <= kFewMarked)
+        {
+            for (uint64_t lanes; (lanes = __ballot(mine != 0)) != 0;)
+            {
+                const int from = __ffsll(static_cast<unsigned long long>(lanes)) - 1;
+                const int bit = __shfl(__ffsll(static_cast<unsigned long long>(mine)) - 1, from, 64);
+                const int i = from + 64 * (bit >> 3);
+                const int row = row0 + m * 32 + i / kChunks, c = col0 + 8 * (i % kChunks) + (bit & 7);
+                const OperandRow a = operand_a(g, row);
+                const float y = row_product(a, operand_w(g, c, false), g.width);
+                const float z = kPair ? row_product(a, operand_w(g, c, true), g.width) : 0.f;
+                if (lane == from)
+                {
+                    store_output<EPI>(g, row, c, y, z);
+                    mine &= mine - 1;
+                }
+            }
+            continue;
+        }
+        const int j = kPair ? lane & 15 : lane & 31;
+        const bool second = kPair && (lane & 16);
+        const OperandRow a = operand_a(g, min(row0 + m * 32 + (lane & 31), g.m - 1));
+#pragma unroll 1
+        for (int n = 0; n < NB; n++)
+        {
+            // A block without marks is left out.
+            bool any = false;
+            for (int i = lane; i < 32 * kChunks; i += 64)
+                any |= i % kChunks / (kBlockCols / 8) == n && (mine >> (i >> 6 << 3) & 0xff) != 0;
+            if (!__any(any))
+                continue;
+            const int c = col0 + n * kBlockCols + j;
+            const f32x16 acc = block_product(a, operand_w(g, min(c, width - 1), second), g.width);
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+            {
+                const float z = kPair ? __shfl_xor(acc[e], 16, 64) : 0.f;
+                const int r = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+                const int i = r * kChunks + (n * kBlockCols + j) / 8;
+                if (!second && (marks[m * 64 + (i & 63)] >> (8 * (i >> 6) + (j & 7)) & 1))
+                    store_output<EPI>(g, row0 + m * 32 + r, c, acc[e], z);
+            }
+        }
     }
 }
 
@@ -357,12 +549,13 @@ __device__ __forceinline__ void run_tile(const GemmProblem& g, const int row0, c
     // Epilogue: 32 rows of a wave's tile at a time through its own part of LDS
     // (accumulator e: column lane % 32, row 8 (e / 4) + 4 (lane / 32) + e % 4),
     // then 8 columns a lane, so that rows are read and written in 16-byte
-    // pieces. Rows and columns with a NaN or an infinity are left to
-    // finish_non_finite.
+    // pieces. SPLIT: an output of which the planes may have lost more than
+    // 2^-22 (its rows' losses) is left to finish_marked.
     constexpr int kPitch = NB * 32 + 4;
     float* part = reinterpret_cast<float*>(smem) + wave * 32 * kPitch;
-    int* meta_row = reinterpret_cast<int*>(smem + kWaves * 32 * kPitch * 4);
-    int* meta_col = meta_row + BM;
+    RowMeta* meta_row = reinterpret_cast<RowMeta*>(smem + kWaves * 32 * kPitch * 4);
+    RowMeta* meta_col = meta_row + BM;
+    uint64_t* marks = reinterpret_cast<uint64_t*>(meta_col + BN) + wave * MB * 64;
     const int width = EPI == kGemmSwiGlu ? g.n >> 1 : g.n;
     arrive<0>();
     if (SPLIT)
@@ -373,7 +566,7 @@ __device__ __forceinline__ void run_tile(const GemmProblem& g, const int row0, c
             meta_col[i] = g.meta_w[weight_row<EPI>(g, col0, i) + (EPI == kGemmSwiGlu && (i & 16) ? width : 0)];
         __syncthreads();
     }
-    int flags = 0;
+    bool marked = false;
     constexpr int kOutCols = EPI == kGemmSwiGlu ? NB * 16 : NB * 32; // of a wave's tile
     constexpr int kChunks = kOutCols / 8;
     const int out_col0 = (EPI == kGemmSwiGlu ? col0 >> 1 : col0) + wn * kOutCols;
@@ -388,6 +581,7 @@ __device__ __forceinline__ void run_tile(const GemmProblem& g, const int row0, c
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        uint64_t mine = 0;
         for (int i = lane; i < 32 * kChunks; i += 64)
         {
             const int r = i / kChunks, ch = i % kChunks;
@@ -404,21 +598,21 @@ __device__ __forceinline__ void run_tile(const GemmProblem& g, const int row0, c
             int bad = 0;
             if (SPLIT)
             {
-                const int ma = meta_row[rl];
-                const int* mc = meta_col + wn * NB * 32 + jl;
+                const RowMeta ma = meta_row[rl];
+                const RowMeta* mc = meta_col + wn * NB * 32 + jl;
 #pragma unroll
                 for (int e = 0; e < 8; e++)
                 {
-                    int f = ma | mc[e];
-                    y[e] = ldexpf(y[e], -row_shift(ma) - row_shift(mc[e]));
+                    bool keep = fabsf(y[e]) >= ma.loss + mc[e].loss; // false for NaN
+                    y[e] = ldexpf(y[e], -ma.shift - mc[e].shift);
                     if (EPI == kGemmSwiGlu)
                     {
-                        f |= mc[e + 16];
-                        z[e] = ldexpf(z[e], -row_shift(ma) - row_shift(mc[e + 16]));
+                        keep = keep && fabsf(z[e]) >= ma.loss + mc[e + 16].loss;
+                        z[e] = ldexpf(z[e], -ma.shift - mc[e + 16].shift);
                     }
-                    bad |= f & (kRowNan | kRowInf) ? 1 << e : 0;
+                    bad |= keep ? 0 : 1 << e;
                 }
-                flags |= bad;
+                mine |= static_cast<uint64_t>(bad) << (i >> 6 << 3);
             }
             if (EPI == kGemmSwiGlu)
 #pragma unroll
@@ -451,12 +645,18 @@ __device__ __forceinline__ void run_tile(const GemmProblem& g, const int row0, c
                     if (!(bad >> e & 1))
                         static_cast<float*>(g.out)[at + e] = y[e];
         }
+        if (SPLIT)
+        {
+            marks[m * 64 + lane] = mine;
+            marked |= mine != 0;
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    if (SPLIT && __builtin_expect(__any(flags), 0))
-        finish_non_finite<EPI>(g, row0 + wm * MB * 32, MB * 32, out_col0, kOutCols);
+    if constexpr (SPLIT)
+        if (__builtin_expect(__any(marked), 0))
+            finish_marked<EPI, MB, NB>(g, marks, row0 + wm * MB * 32, out_col0);
 }
 
 // Both problems' tiles: BM x BN for the video rows, TM x TN for the text rows,
@@ -541,7 +741,6 @@ __global__ __launch_bounds__(kSplitThreads) void split_rows_kernel(const SplitLa
     char* out = static_cast<char*>(s.out) + static_cast<size_t>(row) * p.groups * kStageBytes;
     const int padded = p.groups * kGroup;
     uint32_t max = 0;
-    int flags = 0;
     constexpr int kRegs = CHUNKS > 0 ? CHUNKS : 1;
     float v[kRegs][8];
     if (CHUNKS > 0)
@@ -559,24 +758,22 @@ __global__ __launch_bounds__(kSplitThreads) void split_rows_kernel(const SplitLa
         }
 #pragma unroll
         for (int j = 0; j < kRegs; j++)
-            scan8(v[j], max, flags);
+            scan8(v[j], max);
     }
     else
         for (int k = lane * 8; k < p.width; k += 512)
         {
             load_row8<ALIGNED>(in + k, v[0]);
-            scan8(v[0], max, flags);
+            scan8(v[0], max);
         }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1)
     {
         const uint32_t m = __shfl_xor(max, off, 64);
         max = m > max ? m : max;
-        flags |= __shfl_xor(flags, off, 64);
     }
     const int shift = shift_of(max);
-    if (lane == 0)
-        s.meta[row] = (shift + kShiftBias) | flags;
+    float dropped = 0.f;
     if (CHUNKS > 0)
     {
 #pragma unroll
@@ -584,7 +781,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_rows_kernel(const SplitLa
         {
             const int k = (lane + 64 * j) * 8;
             if (k < padded)
-                store_planes(out, k, v[j], shift);
+                dropped += store_planes(out, k, v[j], shift);
         }
     }
     else
@@ -596,8 +793,13 @@ __global__ __launch_bounds__(kSplitThreads) void split_rows_kernel(const SplitLa
 #pragma unroll
                 for (int e = 0; e < 8; e++)
                     v[0][e] = 0.f;
-            store_planes(out, k, v[0], shift);
+            dropped += store_planes(out, k, v[0], shift);
         }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+        dropped += __shfl_xor(dropped, off, 64);
+    if (lane == 0)
+        s.meta[row] = {shift, row_loss(dropped)};
 }
 
 // A tile shape: video tile, waves, stages, workgroups a CU, and the text tile.
@@ -610,8 +812,8 @@ struct Shape
     static constexpr int kTm = 64, kTn = TN, kTwgm = 2, kTwgn = kWaves / 2, kTstages = TSTAGES;
     static constexpr int kLds = STAGES * (BM + BN) * kStageBytes;
     static_assert(kLds * PER_CU <= 160 * 1024 && TSTAGES * (kTm + TN) * kStageBytes <= kLds, "LDS of a CU");
-    static_assert(kWaves * 32 * (BN / WGN + 4) * 4 + (BM + BN) * 4 <= kLds &&
-                      kWaves * 32 * (TN / kTwgn + 4) * 4 + (kTm + TN) * 4 <= kLds,
+    static_assert(kWaves * 32 * (BN / WGN + 4) * 4 + (BM + BN) * 8 + kWaves * (BM / WGM / 32) * 512 <= kLds &&
+                      kWaves * 32 * (TN / kTwgn + 4) * 4 + (kTm + TN) * 8 + kWaves * 512 <= kLds,
                   "the epilogue's LDS");
 };
 

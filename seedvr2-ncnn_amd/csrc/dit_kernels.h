@@ -10,6 +10,8 @@
 namespace awa
 {
 
+struct RowMeta; // csrc/dit_split.h
+
 // ada[r][c] = emb[c][r / 3][r % 3] + learned[r][c] for the 6 rows (attn
 // shift, scale, gate, mlp shift, scale, gate) of each branch (learned = null:
 // none): the Ada vectors the row kernels below read.
@@ -39,8 +41,10 @@ struct RowNormModulate
     const float* shift;
     const float* scale;
     // Set: out takes the rows' fp16 planes (csrc/dit_split.h, `groups` groups
-    // a row) and meta their shifts instead of the rows themselves.
-    int* meta = nullptr;
+    // a row) and meta what belongs to them; full takes the rows themselves
+    // (stride width) where the planes lose bits.
+    RowMeta* meta = nullptr;
+    float* full = nullptr;
     int groups = 0;
 };
 
@@ -81,12 +85,12 @@ struct SwiGlu
 
 // fp32 rows split into fp16 planes (csrc/dit_gemm.hip): per 32 values of a
 // row 64 bytes of hi and 64 bytes of lo, rows padded with zeros to a whole
-// number of such groups; meta[row] holds the row's shift and flags.
+// number of such groups, and each row's meta (csrc/dit_split.h).
 struct SplitRows
 {
     const float* in; // [rows][width], contiguous
     void* out;       // [rows][groups][128 bytes]
-    int* meta;       // [rows]
+    RowMeta* meta;   // [rows]
     int rows;
 };
 
@@ -105,8 +109,15 @@ struct GemmProblem
     const void* a;
     const void* w;
     const void* w2;    // SwiGLU: the weight of the second half of the columns
-    const int* meta_a; // split: shifts and flags of A's rows and the weights'
-    const int* meta_w;
+    // split: the meta of A's rows and the weights' (w, then w2), and the fp32
+    // operands, rows of `width` values at any 4-byte address: the weights', and
+    // A's at least for the rows that lose bits as planes.
+    const RowMeta* meta_a;
+    const RowMeta* meta_w;
+    const float* full_a;
+    const float* full_w;
+    const float* full_w2;
+    int width;
     uint32_t lda, ldw; // row strides in bytes, multiples of 16
     int m, n, stages;
     uint32_t last_bytes; // bf16: bytes of a row in its last stage

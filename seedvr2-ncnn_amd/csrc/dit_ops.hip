@@ -124,29 +124,22 @@ __global__ __launch_bounds__(kRowThreads) void ada_prepare_kernel(const AdaPrepa
 
 constexpr int kRowChunks = 4; // chunks of 8 a thread keeps in registers (rows up to 8192 wide)
 
-// Largest value and the union of flags over the workgroup.
-__device__ __forceinline__ void block_max(uint32_t& max, int& flags, uint32_t* red)
+// Largest value over the workgroup.
+__device__ __forceinline__ uint32_t block_max(uint32_t max, uint32_t* red)
 {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1)
     {
         const uint32_t m = __shfl_xor(max, off, 64);
         max = m > max ? m : max;
-        flags |= __shfl_xor(flags, off, 64);
     }
-    const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0)
-    {
-        red[wave] = max;
-        red[4 + wave] = static_cast<uint32_t>(flags);
-    }
+        red[threadIdx.x >> 6] = max;
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < 4; w++)
-    {
         max = red[w] > max ? red[w] : max;
-        flags |= static_cast<int>(red[4 + w]);
-    }
+    return max;
 }
 
 // y = rmsnorm(x) * (scale_a + scale_b) + (shift_a + shift_b), one workgroup
@@ -160,7 +153,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const Row
     const int video_rows = pair.branch[0].rows;
     const RowNormModulate& p = pair.branch[static_cast<int>(blockIdx.x) < video_rows ? 0 : 1];
     __shared__ float red[4];
-    __shared__ uint32_t red_max[8];
+    __shared__ uint32_t red_max[4];
     const long long row = static_cast<int>(blockIdx.x) < video_rows ? blockIdx.x : blockIdx.x - video_rows;
     const int chunks = p.width / 8;
     const long long base_in = row * p.in_stride;
@@ -182,7 +175,6 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const Row
     const float inv = 1.f / sqrtf(mean + p.eps);
     const long long base_out = row * p.out_stride;
     uint32_t max = 0;
-    int flags = 0;
 #pragma unroll
     for (int j = 0; j < kRowChunks; j++)
     {
@@ -210,7 +202,7 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const Row
         }
         if (PLANES)
         {
-            scan8(y, max, flags);
+            scan8(y, max);
 #pragma unroll
             for (int e = 0; e < 8; e++)
                 v[j][e] = y[e];
@@ -220,17 +212,28 @@ __global__ __launch_bounds__(kRowThreads) void rmsnorm_modulate_kernel(const Row
     }
     if (PLANES)
     {
-        block_max(max, flags, red_max);
-        const int s = shift_of(max);
-        if (threadIdx.x == 0)
-            p.meta[row] = (s + kShiftBias) | flags;
+        const int s = shift_of(block_max(max, red_max));
         char* out = static_cast<char*>(p.out) + row * p.groups * kStageBytes;
+        float dropped = 0.f;
 #pragma unroll
         for (int j = 0; j < kRowChunks; j++)
         {
             const int k = (threadIdx.x + j * kRowThreads) * 8;
             if (k < p.groups * kGroup)
-                store_planes(out, k, v[j], s);
+                dropped += store_planes(out, k, v[j], s);
+        }
+        dropped = block_sum(dropped, red);
+        if (threadIdx.x == 0)
+            p.meta[row] = {s, row_loss(dropped)};
+        if (dropped == 0.f)
+            return;
+        float* full = p.full + row * p.width;
+#pragma unroll
+        for (int j = 0; j < kRowChunks; j++)
+        {
+            const int k = (threadIdx.x + j * kRowThreads) * 8;
+            if (k < p.width)
+                store8(full, k, 4, v[j]);
         }
     }
 }

@@ -34,6 +34,7 @@
 
 #include "awa_internal.h"
 #include "dit_kernels.h"
+#include "dit_split.h"
 #include "seedvr2_awa.h"
 
 // One GEMM shape's hipBLASLt descriptors and its algorithm: the fastest of
@@ -59,11 +60,11 @@ struct awa_dit_block
     // the branch's Ada vectors [6][hidden] fp32.
     void* ws[2][7] = {};
     float* ada[2] = {nullptr, nullptr};
-    // Split GEMMs (fp32 blocks of enough rows): fp16 planes and shifts of the
+    // Split GEMMs (fp32 blocks of enough rows): fp16 planes and row meta of the
     // activations and of one weight at a time, per branch.
     bool split = false;
-    void* planes[2][2] = {};   // [branch][activations, weight]
-    int* shifts[2][2] = {};
+    void* planes[2][2] = {};         // [branch][activations, weight]
+    awa::RowMeta* meta[2][2] = {};
 };
 
 namespace
@@ -114,10 +115,10 @@ void release(awa_dit_block* b)
         {
             if (b->planes[br][k])
                 (void)hipFree(b->planes[br][k]);
-            if (b->shifts[br][k])
-                (void)hipFree(b->shifts[br][k]);
+            if (b->meta[br][k])
+                (void)hipFree(b->meta[br][k]);
             b->planes[br][k] = nullptr;
-            b->shifts[br][k] = nullptr;
+            b->meta[br][k] = nullptr;
         }
     for (float*& p : b->ada)
     {
@@ -387,18 +388,19 @@ int allocate_split(awa_dit_block* b, long long hd)
                 p = static_cast<std::remove_reference_t<decltype(p)>>(m);
         };
         get(b->ada[br], static_cast<size_t>(6) * d.hidden * sizeof(float));
+        get(b->ws[br][kNorm], M * d.hidden * 4);
         get(b->ws[br][kQkv], M * 3 * hd * 4);
         get(b->ws[br][kAtt], M * hd * 4);
         get(b->ws[br][kResid], M * d.hidden * 4);
         get(b->ws[br][kHidden], M * d.mlp_hidden * 4);
         get(b->planes[br][0], M * std::max({gh, ga, gm}) * 128);
-        get(b->shifts[br][0], M * sizeof(int));
+        get(b->meta[br][0], M * sizeof(awa::RowMeta));
         get(b->planes[br][1], std::max({static_cast<size_t>(3 * hd) * gh, static_cast<size_t>(d.hidden) * ga,
                                         static_cast<size_t>(2) * d.mlp_hidden * gh,
                                         static_cast<size_t>(d.hidden) * gm}) * 128);
-        get(b->shifts[br][1],
+        get(b->meta[br][1],
             static_cast<size_t>(std::max({3 * hd, static_cast<long long>(d.hidden), 2LL * d.mlp_hidden})) *
-                sizeof(int));
+                sizeof(awa::RowMeta));
         if (!ok)
             return fail(AWA_ERR_ALLOC, "DiT block workspace allocation failed");
     }
@@ -467,19 +469,23 @@ int gemm_step(awa_dit_block* b, int buf, const void* const (&w)[2], const void* 
             continue;
         }
         if (buf != kNorm)
-            s.part[2 * br + 1] = {static_cast<const float*>(b->ws[br][buf]), b->planes[br][0], b->shifts[br][0], q.m};
+            s.part[2 * br + 1] = {static_cast<const float*>(b->ws[br][buf]), b->planes[br][0], b->meta[br][0], q.m};
         const size_t pitch = static_cast<size_t>(groups) * 128;
         const int first = w2[br] ? n / 2 : n;
         char* planes = static_cast<char*>(b->planes[br][1]);
-        s.part[2 * br] = {static_cast<const float*>(w[br]), planes, b->shifts[br][1], first};
+        s.part[2 * br] = {static_cast<const float*>(w[br]), planes, b->meta[br][1], first};
         if (w2[br])
-            s.part[2 * br + 1] = {static_cast<const float*>(w2[br]), planes + pitch * first, b->shifts[br][1] + first,
+            s.part[2 * br + 1] = {static_cast<const float*>(w2[br]), planes + pitch * first, b->meta[br][1] + first,
                                   n - first};
         q.a = b->planes[br][0];
         q.w = planes;
         q.w2 = planes + pitch * first;
-        q.meta_a = b->shifts[br][0];
-        q.meta_w = b->shifts[br][1];
+        q.meta_a = b->meta[br][0];
+        q.meta_w = b->meta[br][1];
+        q.full_a = static_cast<const float*>(b->ws[br][buf]);
+        q.full_w = static_cast<const float*>(w[br]);
+        q.full_w2 = static_cast<const float*>(w2[br]);
+        q.width = k;
         q.lda = q.ldw = static_cast<uint32_t>(pitch);
         q.stages = groups;
     }
@@ -519,7 +525,8 @@ int forward_grouped(awa_dit_block* b, const awa_dit_branch_weights* const (&W)[2
             nm.eps = d.norm_eps;
             nm.shift = modulate ? b->ada[br] + static_cast<size_t>(shift_row) * hidden : nullptr;
             nm.scale = modulate ? b->ada[br] + static_cast<size_t>(shift_row + 1) * hidden : nullptr;
-            nm.meta = b->split ? b->shifts[br][0] : nullptr;
+            nm.meta = b->split ? b->meta[br][0] : nullptr;
+            nm.full = b->split ? static_cast<float*>(b->ws[br][kNorm]) : nullptr;
             nm.groups = groups_of(hidden);
         }
         return awa::launch_rmsnorm_modulate(pair, stream);
