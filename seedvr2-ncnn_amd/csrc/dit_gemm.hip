@@ -58,7 +58,7 @@ typedef __attribute__((address_space(3))) char lds_char;
 __device__ __forceinline__ void load_to_lds(const char* base, uint32_t offset, uint32_t lds)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-                 : "memory");
+                 : "memory", "m0");
 }
 
 // Waits for all but the N latest loads of the wave and for its LDS reads, then
