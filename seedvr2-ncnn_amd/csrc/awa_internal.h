@@ -37,3 +37,22 @@ int forward_fused(const awa_plan* plan, const awa_blob* video_qkv, const awa_blo
 int noalloc_setup();
 
 } // namespace awa
+
+// One GEMM step of the DiT block (csrc/dit_gemm.hip) on device operands, with
+// the tile shape given (tests; tile < 0: the estimate's, returned in tile).
+// rows[1] = 0: no text problem. Rows are contiguous; split makes the fp16 planes
+// in memory of its own and waits for the stream.
+struct awa_gemm_step
+{
+    int split, tile, epilogue, n, k;
+    int rows[2], twice[2];
+    const void *a[2], *w[2], *w2[2], *residual[2];
+    const float *bias[2], *gate[2];
+    void* out[2];
+};
+
+extern "C" int awa_gemm_step_run(awa_gemm_step* step, void* stream);
+
+// Whether awa_dit_block_forward runs the block's GEMMs on the library (tests).
+extern "C" int awa_dit_block_on_library(const awa_dit_block* block, const awa_dit_branch_weights* video_weights,
+                                        const awa_dit_branch_weights* text_weights);

@@ -857,7 +857,7 @@ struct Tile
     } cost[2]; // bf16, split
 };
 
-constexpr Tile kTiles[] = {
+constexpr Tile kTiles[kGemmTiles] = {
     {256, 256, {{4.9f, 3.3f, 0.f, 52.6f}, {6.8f, 0.6f, 64.f, 77.1f}}},
     {256, 192, {{0.4f, 0.f, 23.5f, 40.2f}, {6.4f, 28.7f, 81.5f, 68.2f}}},
     {128, 256, {{3.6f, 2.5f, 0.f, 32.6f}, {6.1f, 12.5f, 18.7f, 53.9f}}},
@@ -869,26 +869,9 @@ constexpr Tile kTiles[] = {
 };
 
 template <bool SPLIT>
-hipError_t launch_kind(const GemmLaunch& p, hipStream_t stream)
+hipError_t launch_kind(const GemmLaunch& p, int tile, hipStream_t stream)
 {
-    const GemmProblem& v = p.problem[0];
-    int best = 0;
-    float least = 0.f;
-    for (int i = 0; i < static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0])); i++)
-    {
-        const Tile& t = kTiles[i];
-        const long long tiles = ((v.m + t.bm - 1LL) / t.bm) * ((v.n + t.bn - 1LL) / t.bn);
-        const float k = static_cast<float>(v.stages) * (SPLIT ? 32 : 64) / 2560;
-        const auto& c = t.cost[SPLIT];
-        const float cost = c.start + k * (c.stage + c.share * static_cast<float>(tiles) / kCus +
-                                          c.round * static_cast<float>((tiles + kCus - 1) / kCus));
-        if (i == 0 || cost < least)
-        {
-            best = i;
-            least = cost;
-        }
-    }
-    switch (best)
+    switch (tile)
     {
     case 0:
         return launch_epilogue<Shape<SPLIT, 256, 256, 2, 4, 2, 1, 256, 3>>(p, stream);
@@ -911,12 +894,37 @@ hipError_t launch_kind(const GemmLaunch& p, hipStream_t stream)
 
 } // namespace
 
-hipError_t launch_gemm(const GemmLaunch& p, bool split, hipStream_t stream)
+int gemm_tile(const GemmLaunch& p, bool split)
 {
     const GemmProblem& v = p.problem[0];
-    if (v.m <= 0 || v.n <= 0 || v.n % 8 || v.stages <= 0 || (p.epilogue == kGemmSwiGlu && v.n % 16))
+    int best = 0;
+    float least = 0.f;
+    for (int i = 0; i < kGemmTiles; i++)
+    {
+        const Tile& t = kTiles[i];
+        const long long tiles = ((v.m + t.bm - 1LL) / t.bm) * ((v.n + t.bn - 1LL) / t.bn);
+        const float k = static_cast<float>(v.stages) * (split ? 32 : 64) / 2560;
+        const auto& c = t.cost[split];
+        const float cost = c.start + k * (c.stage + c.share * static_cast<float>(tiles) / kCus +
+                                          c.round * static_cast<float>((tiles + kCus - 1) / kCus));
+        if (i == 0 || cost < least)
+        {
+            best = i;
+            least = cost;
+        }
+    }
+    return best;
+}
+
+hipError_t launch_gemm(const GemmLaunch& p, bool split, hipStream_t stream, int tile)
+{
+    const GemmProblem& v = p.problem[0];
+    if (v.m <= 0 || v.n <= 0 || v.n % 8 || v.stages <= 0 || (p.epilogue == kGemmSwiGlu && v.n % 16) ||
+        tile >= kGemmTiles)
         return hipErrorInvalidValue;
-    return split ? launch_kind<true>(p, stream) : launch_kind<false>(p, stream);
+    if (tile < 0)
+        tile = gemm_tile(p, split);
+    return split ? launch_kind<true>(p, tile, stream) : launch_kind<false>(p, tile, stream);
 }
 
 hipError_t launch_split_rows(const SplitLaunch& p, hipStream_t stream)

@@ -145,7 +145,11 @@ struct GemmLaunch
 };
 
 hipError_t launch_split_rows(const SplitLaunch& p, hipStream_t stream);
-hipError_t launch_gemm(const GemmLaunch& p, bool split, hipStream_t stream);
+// The tile shape (0 .. kGemmTiles - 1) that launch_gemm estimates to be the
+// fastest; tile >= 0 asks for that one instead.
+constexpr int kGemmTiles = 8;
+int gemm_tile(const GemmLaunch& p, bool split);
+hipError_t launch_gemm(const GemmLaunch& p, bool split, hipStream_t stream, int tile = -1);
 
 hipError_t launch_rmsnorm_modulate(const RowNormPair& pair, hipStream_t stream);
 hipError_t launch_gate_residual(const GateResidual& p, hipStream_t stream);

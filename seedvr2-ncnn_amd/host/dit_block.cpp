@@ -822,6 +822,95 @@ int awa_dit_block_forward(awa_dit_block* b, const awa_dit_branch_weights* video_
     return AWA_OK;
 }
 
+int awa_dit_block_on_library(const awa_dit_block* b, const awa_dit_branch_weights* video_w,
+                             const awa_dit_branch_weights* text_w)
+{
+    const awa_dit_branch_weights* const W[2] = {video_w, text_w};
+    return !use_grouped(b, W);
+}
+
+int awa_gemm_step_run(awa_gemm_step* step, void* stream_ptr)
+{
+    if (!step || step->n <= 0 || step->k <= 0 || step->k % 8 || step->epilogue < awa::kGemmStore ||
+        step->epilogue > awa::kGemmSwiGlu)
+        return fail(AWA_ERR_INVALID, "invalid GEMM step");
+    const hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
+    const awa_gemm_step& d = *step;
+    const bool pair = d.epilogue == awa::kGemmSwiGlu;
+    const int groups = groups_of(d.k), first = pair ? d.n / 2 : d.n;
+    const size_t pitch = static_cast<size_t>(groups) * 128;
+    awa::GemmLaunch g{};
+    g.epilogue = d.epilogue;
+    awa::SplitLaunch s[2]{};
+    std::vector<void*> buffers;
+    auto get = [&](size_t bytes) {
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess)
+            return static_cast<char*>(nullptr);
+        buffers.push_back(p);
+        return static_cast<char*>(p);
+    };
+    bool ok = true;
+    for (int br = 0; br < 2; br++)
+    {
+        awa::GemmProblem& q = g.problem[br];
+        q.m = d.rows[br];
+        if (q.m <= 0)
+            continue;
+        q.n = d.n;
+        q.a = d.a[br];
+        q.w = d.w[br];
+        q.w2 = d.w2[br];
+        q.lda = q.ldw = static_cast<uint32_t>(d.k) * 2;
+        q.stages = (d.k + 63) / 64;
+        q.last_bytes = static_cast<uint32_t>(d.k - (q.stages - 1) * 64) * 2;
+        q.out = d.out[br];
+        q.ldo = q.ldr = first;
+        q.bias = d.bias[br];
+        q.gate = d.gate[br];
+        q.residual = d.residual[br];
+        q.twice = d.twice[br];
+        if (!d.split)
+            continue;
+        char *pa = get(pitch * q.m), *pw = get(pitch * d.n);
+        awa::RowMeta* ma = reinterpret_cast<awa::RowMeta*>(get(sizeof(awa::RowMeta) * q.m));
+        awa::RowMeta* mw = reinterpret_cast<awa::RowMeta*>(get(sizeof(awa::RowMeta) * d.n));
+        ok = ok && pa && pw && ma && mw;
+        if (!ok)
+            break;
+        q.full_a = static_cast<const float*>(d.a[br]);
+        q.full_w = static_cast<const float*>(d.w[br]);
+        q.full_w2 = static_cast<const float*>(d.w2[br]);
+        s[br].width = q.width = d.k;
+        s[br].groups = q.stages = groups;
+        s[br].part[0] = {q.full_a, pa, ma, q.m};
+        s[br].part[1] = {q.full_w, pw, mw, first};
+        if (pair)
+            s[br].part[2] = {q.full_w2, pw + pitch * first, mw + first, d.n - first};
+        q.a = pa;
+        q.w = pw;
+        q.w2 = pw + pitch * first;
+        q.meta_a = ma;
+        q.meta_w = mw;
+        q.lda = q.ldw = static_cast<uint32_t>(pitch);
+    }
+    hipError_t e = ok ? hipSuccess : hipErrorOutOfMemory;
+    for (int br = 0; br < 2 && e == hipSuccess; br++)
+        if (s[br].width > 0)
+            e = awa::launch_split_rows(s[br], stream);
+    if (e == hipSuccess)
+    {
+        if (d.tile < 0)
+            step->tile = awa::gemm_tile(g, d.split != 0);
+        e = awa::launch_gemm(g, d.split != 0, stream, step->tile);
+    }
+    if (!buffers.empty())
+        (void)hipStreamSynchronize(stream);
+    for (void* p : buffers)
+        (void)hipFree(p);
+    return e == hipSuccess ? AWA_OK : fail_hip(e, "GEMM step");
+}
+
 } // extern "C"
 
 // ---- The block loop: DitStackSession::run (src/dit/dit_stack.cpp:931-982) ----
