@@ -53,6 +53,9 @@ struct awa_gemm_step
 
 extern "C" int awa_gemm_step_run(awa_gemm_step* step, void* stream);
 
+// The estimate's tile shape for a step (no device is touched).
+extern "C" int awa_gemm_step_tile(const awa_gemm_step* step);
+
 // Whether awa_dit_block_forward runs the block's GEMMs on the library (tests).
 extern "C" int awa_dit_block_on_library(const awa_dit_block* block, const awa_dit_branch_weights* video_weights,
                                         const awa_dit_branch_weights* text_weights);

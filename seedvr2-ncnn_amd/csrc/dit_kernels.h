@@ -147,7 +147,7 @@ struct GemmLaunch
 hipError_t launch_split_rows(const SplitLaunch& p, hipStream_t stream);
 // The tile shape (0 .. kGemmTiles - 1) that launch_gemm estimates to be the
 // fastest; tile >= 0 asks for that one instead.
-constexpr int kGemmTiles = 8;
+constexpr int kGemmTiles = 7;
 int gemm_tile(const GemmLaunch& p, bool split);
 hipError_t launch_gemm(const GemmLaunch& p, bool split, hipStream_t stream, int tile = -1);
 

@@ -829,6 +829,19 @@ int awa_dit_block_on_library(const awa_dit_block* b, const awa_dit_branch_weight
     return !use_grouped(b, W);
 }
 
+int awa_gemm_step_tile(const awa_gemm_step* step)
+{
+    awa::GemmLaunch g{};
+    for (int br = 0; br < 2; br++)
+    {
+        awa::GemmProblem& q = g.problem[br];
+        q.m = step->rows[br];
+        q.n = q.m > 0 ? step->n : 0;
+        q.stages = step->split ? groups_of(step->k) : (step->k + 63) / 64;
+    }
+    return awa::gemm_tile(g, step->split != 0);
+}
+
 int awa_gemm_step_run(awa_gemm_step* step, void* stream_ptr)
 {
     if (!step || step->n <= 0 || step->k <= 0 || step->k % 8 || step->epilogue < awa::kGemmStore ||
@@ -901,7 +914,7 @@ int awa_gemm_step_run(awa_gemm_step* step, void* stream_ptr)
     if (e == hipSuccess)
     {
         if (d.tile < 0)
-            step->tile = awa::gemm_tile(g, d.split != 0);
+            step->tile = awa_gemm_step_tile(step);
         e = awa::launch_gemm(g, d.split != 0, stream, step->tile);
     }
     if (!buffers.empty())
