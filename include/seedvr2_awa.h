@@ -326,18 +326,19 @@ int awa_stack_block_flops(const awa_stack* stack, double* flops);
  * with a NaN or an infinity: those reach the outputs they reach in fp32. A block
  * whose data mark many outputs takes longer, up to about twice the time of
  * the library's fp32 GEMMs. Equal shapes give equal bits in every process.
- * Library GEMMs (hipBLASLt) serve fp32 blocks of fewer than 320 video rows, bf16
- * blocks of more than 5000 video rows at hidden > 1536, operands past 4 GiB
- * and bf16 weights off 16-byte addresses. There the first GEMM of each shape in
- * the process times hipBLASLt's candidate algorithms on the caller's operands
- * and stream, waiting for the stream once (not under graph capture, where the
- * heuristic's first is taken for that call); its choice then holds for every
- * block and stack object of the process, and another process may choose
- * otherwise (last bits). With the environment variable
- * SEEDVR2_GEMM_HEURISTIC=1 the heuristic's first algorithm is taken for every
- * shape, without timing. An fp32 block on split GEMMs keeps planes of its largest
- * weight, 4 bytes a value and branch. A block or stack object is used by one
- * thread at a time. */
+ * Library GEMMs (hipBLASLt) serve fp32 blocks of fewer than 320 video rows (one
+ * more for every 40 of hidden beyond 2560), bf16 blocks of more than 5000 video
+ * rows at hidden > 1536, bf16 weights off 16-byte addresses, and blocks whose
+ * largest row count (tokens or weight rows) times their largest width reaches
+ * 2^30. There the first GEMM of each shape in the process times hipBLASLt's
+ * candidate algorithms on the caller's operands and stream, waiting for the
+ * stream once (not under graph capture, where the heuristic's first is taken for
+ * that call); its choice then holds for every block and stack object of the
+ * process, and another process may choose otherwise (last bits). With the
+ * environment variable SEEDVR2_GEMM_HEURISTIC=1 the heuristic's first algorithm
+ * is taken for every shape, without timing. An fp32 block on split GEMMs keeps
+ * planes of its largest weight, 4 bytes a value and branch. A block or stack
+ * object is used by one thread at a time. */
 typedef struct awa_dit_block_desc {
     int source_t, source_h, source_w;    /* token grid */
     int windows_t, windows_h, windows_w; /* window counts (params 3/4/5) */

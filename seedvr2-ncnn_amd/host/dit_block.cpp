@@ -325,14 +325,20 @@ int groups_of(long long width)
 
 // fp32 blocks of at least this many video rows run their GEMMs on split
 // operands; below, the pass that splits the weights (8 bytes an element, about
-// 230 us of a block at hidden 2560, SwiGLU 6912) costs more than it saves.
-// Whole fp32 block, library GEMMs against split ones: 144 rows 456 / 522 us,
-// 256 rows 559 / 546, 384 rows 708 / 621, 512 rows 826 / 671, 1000 rows 1399 / 916,
-// 2304 rows 2851 / 1378, 4600 rows 5525 / 2438; hidden 1024 and 512 rows 233 / 183.
-constexpr int kSplitMinRows = 320;
+// 230 us of a block at hidden 2560, SwiGLU 6912) costs more than it saves. The
+// rows where both take the same time, whole fp32 block on library GEMMs against
+// split ones, at most about 140 at hidden 1024 and 1536, 190 at 2048 and 270 at
+// 2560 (256 rows 538 / 560 us, 324 rows 705 / 625), 320 at 3072 and 3840, 370 at 5120
+// (324 rows 2025 / 2125, 400 rows 2498 / 2261), 440 at 8192 (400 rows 5746 / 6013, 480
+// rows 6475 / 6060): one line above them all, with the width beyond 2560.
+// Well above it: 2304 rows at hidden 2560 2851 / 1378, 4600 rows 5525 / 2438.
+int split_min_rows(int hidden)
+{
+    return 320 + std::max(0, hidden - 2560) / 40;
+}
 
 // The kernel addresses its operands (at most 4 bytes a value) with 32-bit byte
-// offsets.
+// offsets; the most rows of any operand by the largest width stand for them all.
 bool addressable(const awa_dit_block* b, long long hd)
 {
     const awa_dit_block_desc& d = b->desc;
@@ -344,16 +350,17 @@ bool addressable(const awa_dit_block* b, long long hd)
 
 bool use_split(const awa_dit_block* b, long long hd)
 {
-    return b->desc.precision == AWA_COMPUTE_F32 && b->tokens[0] >= kSplitMinRows && addressable(b, hd);
+    return b->desc.precision == AWA_COMPUTE_F32 && b->tokens[0] >= split_min_rows(b->desc.hidden) && addressable(b, hd);
 }
 
 // bf16 blocks run on the grouped GEMMs up to this many video rows, narrow ones
 // at any: beyond, the library's larger wave tiles gain more per MFMA than the
 // fused epilogues and the shared launch save. Whole bf16 block, library against
-// grouped GEMMs, hidden 2560: 81 rows (hidden 1024) 144 / 70 us, 256 rows
-// 234 / 185, 512 rows 270 / 243, 1000 rows 338 / 338, 2304 rows 532 / 496, 4600 rows
-// 826 / 824, 6400 rows 1136 / 1200, 9200 rows 1494 / 1520; hidden 1536, 9200 rows
-// 776 / 660; hidden 1024, 6400 rows 398 / 282.
+// grouped GEMMs, hidden 2560: 256 rows 235 / 168 us, 512 rows 274 / 221, 972 rows
+// 339 / 302, 2304 rows 532 / 482, 3078 rows 699 / 673, 4446 rows 852 / 862, 4788 rows
+// 913 / 910, 6250 rows 1039 / 1072, 9000 rows 1476 / 1496 (but 5400 rows 990 / 953 and
+// 23400 rows 4223 / 3819); 9000 rows at hidden 2048 1141 / 1103, 1792 874 / 858, 1536
+// 738 / 625; 6400 rows at hidden 1024 398 / 282.
 constexpr int kGroupedMaxRows = 5000;
 constexpr int kGroupedNarrow = 1536;
 

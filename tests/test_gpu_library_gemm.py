@@ -1,6 +1,6 @@
 """DiT blocks on either side of the rules that choose between the GEMMs of
-csrc/dit_gemm.hip and the library's (fp32: 320 video rows; bf16: 5000 video rows at
-hidden > 1536), and the library path in each form it takes: shifted, last
+csrc/dit_gemm.hip and the library's (fp32: 320 video rows, 384 at hidden 5120; bf16:
+5000 video rows at hidden > 1536), and the library path in each form it takes: shifted, last
 block, MLP weights stored apart and back to back. Against the oracle block
 with the block tests' tolerances, fp32 1e-5 and bf16 2e-2 of the largest value."""
 
@@ -19,6 +19,7 @@ from test_gpu_split_gemm import off, weights
 pytestmark = pytest.mark.gpu
 
 FP32 = dict(heads=2, hidden=512, mlp=1384)
+WIDE = dict(heads=1, hidden=5120, mlp=64)
 BF16 = dict(heads=1, hidden=1544, mlp=200)
 
 
@@ -51,6 +52,8 @@ def run(args, es, last, adjacent, heads, hidden, mlp):
     (4, (1, 11, 29), FP32, True),                     # 319 rows
     (4, (1, 16, 20), FP32, False),                    # 320
     (4, (1, 1, 9), FP32, True),
+    (4, (1, 19, 20), WIDE, True),                     # 380 rows, where the library is the faster
+    (4, (2, 16, 12), WIDE, False),                    # 384
     (2, (5, 25, 40), BF16, False),                    # 5000
     (2, (6, 28, 30), BF16, True),                     # 5040
     (2, (6, 28, 30), dict(BF16, hidden=1536), False),
