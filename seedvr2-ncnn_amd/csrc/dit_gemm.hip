@@ -80,8 +80,11 @@ __device__ __forceinline__ int weight_row(const GemmProblem& g, int col0, int j)
     return min((col0 >> 1) + (j >> 5) * 16 + (j & 15), (g.n >> 1) - 1);
 }
 
-// silu(a) * b; to be rounded to bf16 (fast) on the hardware's exp2 and
-// reciprocal, which are good to 2^-20 here.
+// silu(a) * b; to be rounded to bf16 (2^-9) on the hardware's exp2 and
+// reciprocal, in which a log2(e) is rounded: silu is off by at most 2^-20.8 for
+// a >= -10, 2^-19 to -40 and 2^-18 to -87.3, below which it is zero (expf and a
+// division: 2^-22.5 to -88.7). The 33-frame bf16 block is 3.69e-3 off its 64-bit
+// result with either, and 1.9 % slower with expf and the division.
 template <bool FAST>
 __device__ __forceinline__ float silu_mul(float a, float b)
 {
@@ -849,12 +852,11 @@ hipError_t launch_epilogue(const GemmLaunch& p, hipStream_t stream)
 // chip and leave the last round full, large ones read less LDS and L2 per MFMA;
 // which wins lies at other rows for every width, so the estimate decides. It was
 // fitted at 240 launches (81 .. 9200 video rows, 64 text rows, the four GEMMs of
-// hidden 1024, 2048 and 2560; 132 bf16, 108 split; weights from HBM; the 2304-row
-// bf16 SwiGLU as it runs within the block, where 256 x 256 is the faster): it
-// takes the best shape, or one within 0.5 % of it, at 202, is 0.6 % behind the
-// best on average, and at worst 20 % in bf16 (420 x 6144, K 2048: 31 us) and 6 %
-// split. 280 launches of 37 other row counts, not fitted: 0.9 % behind on average, at
-// worst 15 % in bf16 and 11 % split.
+// hidden 1024, 2048 and 2560; 132 bf16, 108 split; weights from HBM): it takes the
+// best shape, or one within 0.5 % of it, at 202, is 0.5 % behind the best on
+// average, and at worst 20 % in bf16 (420 x 6144, K 2048: 31 us) and 6 % split. At 280
+// launches that were not fitted (other rows of the same widths) it is 0.9 %
+// behind on average, at worst 15 % in bf16 and 11 % split.
 struct Tile
 {
     int bm, bn, tn;
@@ -865,13 +867,13 @@ struct Tile
 };
 
 constexpr Tile kTiles[kGemmTiles] = {
-    {256, 256, 256, {{3.f, 14.6f, 24.5f, 37.7f}, {5.2f, 17.7f, 141.2f, 54.2f}}},
-    {256, 192, 128, {{4.1f, 4.6f, 25.4f, 31.1f}, {13.5f, 0.f, 103.7f, 46.7f}}},
-    {128, 256, 256, {{2.7f, 5.1f, 5.7f, 32.3f}, {10.f, 3.f, 47.7f, 51.2f}}},
-    {128, 192, 192, {{7.f, 13.8f, 6.8f, 17.7f}, {5.1f, 24.9f, 24.3f, 41.7f}}}, // two workgroups a CU
+    {256, 256, 256, {{3.3f, 14.1f, 24.5f, 37.9f}, {5.2f, 17.7f, 141.2f, 54.2f}}},
+    {256, 192, 128, {{4.5f, 4.1f, 23.8f, 32.3f}, {13.5f, 0.f, 103.7f, 46.7f}}},
+    {128, 256, 256, {{2.7f, 5.4f, 6.2f, 31.9f}, {10.f, 3.f, 47.7f, 51.2f}}},
+    {128, 192, 192, {{7.3f, 13.6f, 7.1f, 17.4f}, {5.1f, 24.9f, 24.3f, 41.7f}}}, // two workgroups a CU
     {128, 192, 192, {{6.4f, 0.3f, 5.7f, 27.7f}, {8.2f, 0.f, 40.5f, 41.f}}},     // one, deeper
-    {64, 128, 128, {{1.4f, 8.5f, 4.3f, 11.4f}, {1.7f, 11.3f, 13.1f, 24.f}}},
-    {64, 64, 64, {{2.5f, 4.8f, 1.5f, 9.5f}, {0.f, 14.4f, 6.1f, 15.2f}}},
+    {64, 128, 128, {{1.5f, 8.5f, 4.3f, 11.4f}, {1.7f, 11.3f, 13.1f, 24.f}}},
+    {64, 64, 64, {{2.5f, 4.8f, 1.4f, 9.5f}, {0.f, 14.4f, 6.1f, 15.2f}}},
 };
 
 template <bool SPLIT>
