@@ -182,7 +182,8 @@ constexpr long long kDeviceCus = 256;
 // of idle waves cost little. Measured at 24 layers of mixed windows of up to
 // 1720 rows, 4-wave against 8-wave time: 1.28-1.33 where the mean work item
 // has at least 670 keys, 0.93-1.07 at 400-600 keys, 0.86-1.05 below; the
-// 121-frame 720p bf16 layer 4016 / 2776 us, the 49-frame fp32 one 4871 / 3720.
+// 121-frame 720p bf16 layer 4013-4031 / 2686-2802 us across machines, the 49-frame
+// fp32 one 4870-4970 / 3603-3753.
 int attention_variant(int compute, const awa_plan& plan, int heads)
 {
     if (compute == AWA_COMPUTE_F32_MFMA)

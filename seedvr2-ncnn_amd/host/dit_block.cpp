@@ -3,20 +3,23 @@
 // block, src/dit/dit_stack.cpp:951-963):
 //
 //   x_a   = rmsnorm(x) * (1 + ...) Ada "in" (attn)        rmsnorm_modulate kernel
-//   qkv   = x_a W_qkv^T                                    GEMM (hipBLASLt)
+//   qkv   = x_a W_qkv^T                                    GEMM
 //   att   = AWA(q/k RMSNorm(qkv))                          awa_forward_qknorm
-//   y     = (att W_out^T + b) * gate_attn + x              GEMM + gate_residual kernel
+//   y     = (att W_out^T + b) * gate_attn + x              GEMM with this epilogue
 //   x_m   = rmsnorm(y) Ada "in" (mlp)                      rmsnorm_modulate kernel
-//   h     = silu(x_m W_gate^T) * (x_m W_in^T)              2 GEMMs into one buffer + swiglu kernel
-//   out   = (h W_mlp^T) * gate_mlp + y                     GEMM + gate_residual kernel
+//   h     = silu(x_m W_gate^T) * (x_m W_in^T)              GEMM with this epilogue
+//   out   = (h W_mlp^T) * gate_mlp + y                     GEMM with this epilogue
 //
 // for the video and the text branch; the last block modulates and runs the
 // MLP on video only and returns text as 2 * y_text. Precision follows the
-// block: fp32 blocks keep fp32 activations, weights and GEMMs; bf16 blocks
-// store activations and GEMM weights in bf16 (round to nearest even) and
-// accumulate in fp32. Parameter vectors (biases, gammas, Ada) are fp32. fp32
-// blocks of enough rows run their GEMMs on split operands (csrc/dit_gemm.hip)
-// with the steps after them in the epilogues (forward_grouped).
+// block: fp32 blocks keep fp32 activations and weights; bf16 blocks store
+// activations and GEMM weights in bf16 (round to nearest even) and accumulate
+// in fp32. Parameter vectors (biases, gammas, Ada) are fp32.
+//
+// forward_grouped runs the GEMMs of csrc/dit_gemm.hip, both branches' in one
+// launch (fp32 on split operands). Where the library's are the faster or must
+// serve (split_min_rows, use_grouped) awa_dit_block_forward runs hipBLASLt GEMMs,
+// one a branch, with the epilogues as the row kernels gate_residual and swiglu.
 #include <hip/hip_runtime.h>
 #include <hipblaslt/hipblaslt.h>
 
