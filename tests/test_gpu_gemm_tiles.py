@@ -57,7 +57,8 @@ def operands(rng, rows, n, k, epilogue, es):
     return op
 
 
-def run(split, tile, epilogue, n, k, branches):
+def run(split, tile, epilogue, n, k, branches, off_16=False):
+    """off_16: the weights one element into their allocations (split only)."""
     es = 4 if split else 2
     step = GemmStep(split=split, tile=tile, epilogue=epilogue, n=n, k=k)
     width = n // 2 if epilogue == SWIGLU else n
@@ -67,8 +68,9 @@ def run(split, tile, epilogue, n, k, branches):
         step.rows[br] = rows
         step.twice[br] = br if epilogue == GATE else 0
         for name, x in op.items():
-            keep.append(to_device(x, 4 if name in ("bias", "gate") else es))
-            getattr(step, name)[br] = keep[-1].ptr
+            moved = off_16 and name in ("w", "w2")
+            keep.append(to_device(np.append(np.float32(0), x) if moved else x, 4 if name in ("bias", "gate") else es))
+            getattr(step, name)[br] = keep[-1].ptr + (es if moved else 0)
         outs.append(A.DeviceBuffer(rows * width * es))
         step.out[br] = outs[-1].ptr
     A.check(A.lib().awa_gemm_step_run(ctypes.byref(step), None), "awa_gemm_step_run")
@@ -142,7 +144,8 @@ def test_every_tile_shape(gpu, split, tile, epilogue):
 @pytest.mark.parametrize("tile", range(len(TILES)))
 def test_outputs_that_planes_cannot_give(gpu, tile, epilogue, kind):
     """Split GEMMs whose rows hold infinities, NaN and values that vanish as
-    planes; some outputs (a few of 32 rows and whole rows of them), and all."""
+    planes; some outputs (a few of 32 rows and whole rows of them), and all.
+    Weights on 16-byte addresses and off them."""
     print(f"case GEMM marked outputs tile={tile} epilogue={epilogue} {kind}", flush=True)
     rng = np.random.default_rng(7 + 10 * tile + epilogue)
     rows, n = size_of(tile, epilogue)
@@ -170,7 +173,7 @@ def test_outputs_that_planes_cannot_give(gpu, tile, epilogue, kind):
             if epilogue == SWIGLU:
                 w[20, 9] = 2.0 ** 58            # silu of a moderate value
                 a[40] *= np.float32(2.0 ** -100)
-        got, _ = run(1, tile, epilogue, n, k, branches)
+        got, _ = run(1, tile, epilogue, n, k, branches, off_16=k == 232)
         for br, (x, op) in enumerate(zip(got, branches)):
             compare(x, op, epilogue, br if epilogue == GATE else 0, 4, f"k={k} branch={br}")
 
